@@ -12,7 +12,8 @@
 //    d2 = (dx*dx + dy*dy) + dz*dz and r = ((double)radius[t_i * ntypes + t_j] + shift_i) + shift_j,
 //    all in IEEE double, and r >= 0 (the exact pair test of the sphere query with a per-pair
 //    radius: HOOMD-style diameter shifting with shift = (diameter - 1) / 2).
-// One thread per row; rows laid out in traversal order put the rows of a wave side by side.
+// The filter runs one thread per row; rows laid out in traversal order put the rows of a wave
+// side by side.  The packing copies groups of four pairs, one per lane.
 // (No counterpart in the reference.)
 #ifndef NEIGHBOR_KERNELS_ROW_FILTER_H_
 #define NEIGHBOR_KERNELS_ROW_FILTER_H_
@@ -96,25 +97,83 @@ __global__ void __launch_bounds__(256) rows_filter(const RowFilterArgs a)
     a.counts_out[q] = kept;
     }
 
+//! Four pairs' worth of row data at any address: the compiler emits one 16-byte (4-byte) access
+//! for the neighbors (image bytes), which global memory takes at 4-byte (1-byte) alignment.
+struct __attribute__((packed, aligned(4))) RowQuad { uint32_t v[4]; };
+struct __attribute__((packed, aligned(1))) ImageQuad { uint32_t v; };
+
 //! Row q = [start[q], start[q] + counts[q]) copied to [offsets[q], offsets[q] + counts[q]) of the
 //! output arrays (CSR rows without gaps, offsets from a scan of counts), and first[e] = i for each
 //! pair e of the row (with neigh and image: the (i, j, image) pair stream).  Any output may be null.
+/*!
+ * A copy, so bound by HBM.  A wave copies the pairs of its 64 rows in groups of four consecutive
+ * pairs of a row, one group per lane: the lanes of a wave then read and write runs of whole rows,
+ * at full lane use whatever the rows' lengths (a lane finds its group's row by bisecting the
+ * wave's running group counts in LDS).  A row's last group starts four before its end, so rows
+ * of four or more pairs take one wide load and store per group and array (the overlap with the
+ * group before is written twice, with the same values); shorter rows go pair by pair.
+ * Measured on 10^6 rows of 79 pairs on average (source rows in Morton order, 0.79 GB moved):
+ * one thread per row took 4571 us (64 rows' lines per load); so, about 225 us (3.5 TB/s).
+ */
 __global__ void __launch_bounds__(256) rows_pack(const unsigned long long* __restrict__ start, const uint32_t* __restrict__ counts,
                                                  const uint32_t n, const uint32_t* __restrict__ query_index,
                                                  const unsigned long long* __restrict__ offsets, const uint32_t* __restrict__ neigh,
                                                  const uint8_t* __restrict__ image, uint32_t* __restrict__ neigh_out,
                                                  uint8_t* __restrict__ image_out, uint32_t* __restrict__ first_out)
     {
+    __shared__ unsigned long long s_group[4][64];       // groups of the wave's rows before each row
+    __shared__ unsigned long long s_from[4][64];
+    __shared__ unsigned long long s_to[4][64];
+    __shared__ uint32_t s_count[4][64];
+    __shared__ uint32_t s_first[4][64];
+    const unsigned int lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
     const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n) return;
-    const uint32_t i = query_index ? query_index[q] : q;
-    const unsigned long long s = start[q], o = offsets[q];
-    const uint32_t c = counts[q];
-    for (uint32_t e = 0; e < c; ++e)
+    const bool valid = q < n;
+    const uint32_t c = valid ? counts[q] : 0u;
+    const unsigned long long g = (static_cast<unsigned long long>(c) + 3ull) / 4ull;
+    unsigned long long incl = g;
+    #pragma unroll
+    for (unsigned int d = 1; d < 64; d <<= 1)
         {
-        if (neigh_out) neigh_out[o + e] = neigh[s + e];
-        if (image_out) image_out[o + e] = image[s + e];
-        if (first_out) first_out[o + e] = i;
+        const unsigned long long y = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += y;
+        }
+    s_group[w][lane] = incl - g;
+    s_from[w][lane] = valid ? start[q] : 0ull;
+    s_to[w][lane] = valid ? offsets[q] : 0ull;
+    s_count[w][lane] = c;
+    s_first[w][lane] = valid && first_out ? (query_index ? query_index[q] : q) : 0u;
+    const unsigned long long total = __shfl(incl, 63, 64);
+    __syncthreads();
+    for (unsigned long long t = lane; t < total; t += 64ull)
+        {
+        // the last row whose groups start at or before t (rows without groups share a start)
+        unsigned int r = 0;
+        #pragma unroll
+        for (unsigned int step = 32; step > 0; step >>= 1)
+            if (s_group[w][r + step] <= t) r += step;
+        const uint32_t cr = s_count[w][r];
+        unsigned long long e = (t - s_group[w][r]) * 4ull;
+        const unsigned long long from = s_from[w][r], to = s_to[w][r];
+        const uint32_t i = s_first[w][r];
+        if (cr >= 4u)
+            {
+            if (e + 4ull > cr) e = cr - 4u;
+            if (neigh_out)
+                *reinterpret_cast<RowQuad*>(neigh_out + to + e) = *reinterpret_cast<const RowQuad*>(neigh + from + e);
+            if (image_out)
+                *reinterpret_cast<ImageQuad*>(image_out + to + e) = *reinterpret_cast<const ImageQuad*>(image + from + e);
+            if (first_out) *reinterpret_cast<RowQuad*>(first_out + to + e) = RowQuad{{i, i, i, i}};
+            }
+        else
+            {
+            for (uint32_t k = 0; k < cr; ++k)
+                {
+                if (neigh_out) neigh_out[to + k] = neigh[from + k];
+                if (image_out) image_out[to + k] = image[from + k];
+                if (first_out) first_out[to + k] = i;
+                }
+            }
         }
     }
 
