@@ -7,14 +7,14 @@
 // traverse() silently returns for an empty tree, no queries or no images and
 // throws std::runtime_error for more than 32 images (LBVHTraverser.h:423-432).
 //
-// Variants (this library): Quantized walks the reference's 16-B records;
-// FloatRope walks 32-B records holding the decoded quantized boxes (same
-// results, no decode work per visit); FloatRopeExact holds the exact node boxes
-// and is meant for ExactSphereQueryOp (with the float SphereQueryOp it reports
-// fewer, tighter hits than the reference); Wave (ExactSphereQueryOp only) walks
-// exact-box records with bucket leaves, one rope path per wave of 64 queries;
-// WaveQuantized is the same walk over decoded quantized boxes, for SphereQueryOp
-// (results identical to Quantized) and ExactSphereQueryOp.
+// Variants (this library): Quantized holds the reference's 16-B records; FloatRope 32-B records
+// with the decoded quantized boxes (same results); FloatRopeExact the exact node boxes, meant for
+// ExactSphereQueryOp (with the float SphereQueryOp it reports fewer, tighter hits than the
+// reference); Wave (ExactSphereQueryOp only) exact-box records with bucket leaves; WaveQuantized
+// the same over decoded quantized boxes, for SphereQueryOp (results identical to Quantized) and
+// ExactSphereQueryOp.  SphereQueryOp in every variant and ExactSphereQueryOp in the wave variants
+// walk by node fronts (kernels/FrontWalk.h); other query ops, and ExactSphereQueryOp in the rope
+// variants, take one rope path per query.
 #ifndef NEIGHBOR_LBVH_TRAVERSER_H_
 #define NEIGHBOR_LBVH_TRAVERSER_H_
 
@@ -26,10 +26,14 @@
 #include "TransformOps.h"
 #include "TranslateOps.h"
 #include "Tunable.h"
+#include "kernels/FrontWalk.h"
 #include "kernels/LBVHTraverse.h"
 
+#include <algorithm>
+#include <memory>
 #include <stdexcept>
 #include <type_traits>
+#include <vector>
 
 namespace neighbor
 {
@@ -191,6 +195,123 @@ class LBVHTraverser : public Tunable<unsigned int>
         template<class TransformOpT>
         void compress(const LaunchParameters& params, const LBVH& lbvh, const TransformOpT& transform);
 
+        //! Workspace that sorts the queries of one launch: used by one stream at a time (done: the
+        //! last launch that reads it).
+        struct QuerySort
+            {
+            shared_array<unsigned int> keys[2], vals[2], work;
+            stream_t stream = nullptr;
+            std::shared_ptr<void> done;     //!< hipEvent_t
+            };
+        //! Bounded: a launch finds its stream's workspace, a free one, or waits for the oldest.
+        static constexpr size_t kQuerySorts = 4;
+        std::vector<QuerySort> m_sorts;
+        size_t m_oldest_sort = 0;
+
+        QuerySort& query_sort(stream_t stream)
+            {
+            for (QuerySort& s : m_sorts)
+                if (s.stream == stream) return s;
+            for (QuerySort& s : m_sorts)
+                {
+                if (hipEventQuery(static_cast<hipEvent_t>(s.done.get())) == hipSuccess)
+                    {
+                    s.stream = stream;
+                    return s;
+                    }
+                (void)hipGetLastError();    // not ready
+                }
+            if (m_sorts.size() < kQuerySorts)
+                {
+                hipEvent_t e;
+                NEIGHBOR_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+                QuerySort s;
+                s.done = std::shared_ptr<void>(static_cast<void*>(e), [](void* p) { (void)hipEventDestroy(static_cast<hipEvent_t>(p)); });
+                s.stream = stream;
+                m_sorts.push_back(s);
+                return m_sorts.back();
+                }
+            QuerySort& s = m_sorts[m_oldest_sort++ % kQuerySorts];
+            NEIGHBOR_HIP_CHECK(hipStreamWaitEvent(stream, static_cast<hipEvent_t>(s.done.get()), 0));
+            s.stream = stream;
+            return s;
+            }
+
+        static bool capturing(stream_t stream)
+            {
+            hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+            const hipError_t e = hipStreamIsCapturing(stream, &status);
+            if (e != hipSuccess) (void)hipGetLastError();
+            return e != hipSuccess || status != hipStreamCaptureStatusNone;
+            }
+
+        //! Queries in the Morton order of their centers in the root box (16 or 24 bits of code).
+        const unsigned int* sorted_queries(QuerySort& s, const float4* spheres, const unsigned int n, stream_t stream)
+            {
+            const unsigned int bits = n <= (1u << 20) ? 16u : 24u;
+            const size_t words = gpu::radix::Workspace::words(n, bits);
+            if (n > s.keys[0].size())
+                for (int i = 0; i < 2; ++i)
+                    {
+                    shared_array<unsigned int>(n, MemoryKind::Device).swap(s.keys[i]);
+                    shared_array<unsigned int>(n, MemoryKind::Device).swap(s.vals[i]);
+                    }
+            if (words > s.work.size()) shared_array<unsigned int>(words, MemoryKind::Device).swap(s.work);
+            const gpu::radix::Workspace ws = gpu::radix::Workspace::carve(s.work.get(), n, bits);
+            const size_t header = gpu::radix::Workspace::header_words(ws.passes);
+            hipLaunchKernelGGL(gpu::radix::kernel::fill_zero, dim3(div_up(header, 256)), dim3(256), 0, stream, ws.hist, header);
+            hipLaunchKernelGGL(gpu::kernel::query_codes, dim3(std::min<unsigned int>(div_up(n, 1024), 2048u)), dim3(256), 0, stream,
+                               spheres, n, m_lbvh_lo.get(), m_lbvh_hi.get(), bits, s.keys[0].get(), ws.hist, ws.passes, ws.status,
+                               static_cast<size_t>(ws.passes) * ws.tiles * gpu::radix::kRadix);
+            const bool alt = gpu::radix::sort_passes(s.keys[0].get(), s.vals[0].get(), s.keys[1].get(), s.vals[1].get(), n, true, ws, stream);
+            return s.vals[alt ? 1 : 0].get();
+            }
+
+        //! The front walk's launch: few queries by teams of four waves, others by one wave per 64.
+        template<class QueryOpT, class OutputOpT, class TranslateOpT, class SourceT>
+        void launch_front(const LaunchParameters& params, const QueryOpT& query, const OutputOpT& out, const TranslateOpT& images,
+                          const unsigned int* order, const unsigned int n_nodes, const SourceT& src)
+            {
+            constexpr bool placed = gpu::kernel::wave::places_rows<OutputOpT>::value;    // whole groups per block
+            // queries in no given order are sorted first: a wave's queries must lie close together
+            QuerySort* sorted = nullptr;
+            if constexpr (!placed)
+                if (!order && query.size() > kSortQueries && !capturing(params.stream))
+                    {
+                    sorted = &query_sort(params.stream);
+                    order = sorted_queries(*sorted, query.spheres, query.size(), params.stream);
+                    }
+            launch_front_in_order(params, query, out, images, order, n_nodes, src);
+            if (sorted) NEIGHBOR_HIP_CHECK(hipEventRecord(static_cast<hipEvent_t>(sorted->done.get()), params.stream));
+            }
+
+        template<class QueryOpT, class OutputOpT, class TranslateOpT, class SourceT>
+        void launch_front_in_order(const LaunchParameters& params, const QueryOpT& query, const OutputOpT& out, const TranslateOpT& images,
+                                   const unsigned int* order, const unsigned int n_nodes, const SourceT& src)
+            {
+            constexpr bool placed = gpu::kernel::wave::places_rows<OutputOpT>::value;
+            constexpr bool teams = !placed && (gpu::kernel::front::Rows<OutputOpT>::kOn || std::is_same<OutputOpT, CountNeighborsOp>::value);
+            const unsigned int n = query.size();
+            if constexpr (teams)
+                if (n <= kTeamQueries)
+                    {
+                    const unsigned int per = n <= kTeamQueries / 4u ? 16u : n <= kTeamQueries / 2u ? 32u : 64u;
+                    hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_team<SourceT, OutputOpT, QueryOpT, TranslateOpT>),
+                                       dim3(div_up(n, per)), dim3(256), 0, params.stream, out, src, m_lbvh_lo.get(), m_lbvh_hi.get(),
+                                       m_bins.get(), m_root, query, images, order, n_nodes, per);
+                    return;
+                    }
+            // tail-split map (wave::tail_block): XCD 0 holds the most groups; the other XCDs'
+            // blocks past their own count exit at once
+            const unsigned int tail = placed ? 0u : m_tail_set || n <= kShortTail ? m_tail_groups : kShortTailGroups;
+            const unsigned int G = div_up(n, 256);
+            const unsigned int x0 = G / 8u + (G % 8u ? 1u : 0u);
+            const dim3 grid = tail ? dim3(8u * (x0 + (m_tail_split - 1u) * std::min(x0, tail))) : dim3(G);
+            hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_front<SourceT, OutputOpT, QueryOpT, TranslateOpT>), grid, dim3(256), 0,
+                               params.stream, out, src, m_lbvh_lo.get(), m_lbvh_hi.get(), m_bins.get(), m_root, query, images, order,
+                               n_nodes, tail, m_tail_split);
+            }
+
         //! Wave walk: defined for ExactSphereQueryOp only.
         template<class QueryOpT, class OutputOpT, class TranslateOpT, class TransformOpT>
         void traverse_wave(const LaunchParameters& params, const LBVH& lbvh, const QueryOpT& query, const OutputOpT& out,
@@ -222,24 +343,9 @@ class LBVHTraverser : public Tunable<unsigned int>
                         throw std::invalid_argument("the visit log records count traversals only");
                         }
                     }
-                if constexpr (gpu::kernel::wave::compactable<OutputOpT, QueryOpT>::value)
-                    {
-                    // tail-split map (wave::tail_block): XCD 0 holds the most groups; the other
-                    // XCDs' blocks past their own count exit at once
-                    const unsigned int G = div_up(query.size(), 256);
-                    const unsigned int x0 = G / 8u + (G % 8u ? 1u : 0u);
-                    const dim3 tgrid = m_tail_groups ? dim3(8u * (x0 + (m_tail_split - 1u) * std::min(x0, m_tail_groups)))
-                                                     : grid;
-                    hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_wave_pairs<OutputOpT, QueryOpT, TranslateOpT, TransformOpT>),
-                                       tgrid, dim3(256), 0, params.stream, out, m_float.get(), lbvh.getSortedPoints().get(),
-                                       lbvh.getPrimitives().get(), m_lbvh_lo.get(), m_lbvh_hi.get(), m_root, query, images,
-                                       transform, order, lbvh.getNNodes(), m_tail_groups, m_tail_split);
-                    }
-                else
-                    hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_wave<OutputOpT, QueryOpT, TranslateOpT, TransformOpT>),
-                                       grid, dim3(256), 0, params.stream, out, m_float.get(), lbvh.getSortedPoints().get(),
-                                       lbvh.getPrimitives().get(), m_lbvh_lo.get(), m_lbvh_hi.get(), m_root, query, images,
-                                       transform, order, lbvh.getNNodes(), nullptr);
+                typedef gpu::kernel::front::BucketSource<TransformOpT> Source;
+                launch_front(params, query, out, images, order, lbvh.getNNodes(),
+                             Source{m_float.get(), lbvh.getSortedPoints().get(), lbvh.getPrimitives().get(), transform, lbvh.getNInternal()});
                 }
             else
                 {
@@ -248,13 +354,26 @@ class LBVHTraverser : public Tunable<unsigned int>
             }
 
         unsigned int m_bucket = 16;
-        //! Tail split of the compacted walks: per XCD, the last m_tail_groups groups of 256 queries
-        //! run as m_tail_split blocks each.  32 groups of four waves are one wave for each SIMD of
-        //! an XCD (32 CUs x 4 SIMDs), the last wave each SIMD receives.  Measured at N=10^6
-        //! (uniform, 27 images, 48 leaves per bucket): exact count 0.452 -> 0.438 ms, placed fill
-        //! 0.632 -> 0.623 ms; 64 or 128 split groups, or blocks of 64 queries, were slower.
+        //! Queries given without an order above which they are sorted first: the sort takes about
+        //! 40 us for few queries and 70 us for 10^6; a count of 1000 queries in random order (27
+        //! images) takes 89 us against 43 in Morton order, of 8000 179 against 71, and of 10^6
+        //! (one rope path per lane) 8.2 ms against 0.64.
+        static constexpr unsigned int kSortQueries = 1024;
+        //! Queries up to which four waves serve 64, 32 or 16 queries together: one wave's chain of
+        //! steps takes longer than the chip needs for all of them.  Exact count and fill of 10,000
+        //! points (27 images): 82 and 115 us with a wave per 64 queries, 48 and 61 with teams for
+        //! 16; of 131,071 points (no images) 90 and 125 us with waves, 201 and 229 with teams.
+        static constexpr unsigned int kTeamQueries = 1u << 16;
+        //! Tail split (wave::tail_block): per XCD, the last m_tail_groups groups of 256 queries run
+        //! as m_tail_split blocks each, so that the waves that start last are shorter.  Exact count
+        //! and fill of 300,007 points: 204 and 297 us with 32 groups, 222 and 329 with none; of 10^6
+        //! points, where the tail is a smaller part, 348 and 581 us with 16 groups, 358 and 597 with
+        //! 32, 356 and 594 with none.
         unsigned int m_tail_groups = 32;
         unsigned int m_tail_split = 2;
+        bool m_tail_set = false;        //!< by setTailSplit: kept for any number of queries
+        static constexpr unsigned int kShortTail = 1u << 19;
+        static constexpr unsigned int kShortTailGroups = 16;
 
     public:
         //! Leaves per bucket of the wave variant (1..64); takes effect at the next compression.
@@ -266,7 +385,7 @@ class LBVHTraverser : public Tunable<unsigned int>
             }
         unsigned int getBucketSize() const { return m_bucket; }
 
-        //! Tail split of the compacted exact walks (counts and pair fills): per XCD, the last
+        //! Tail split of the front walk: per XCD, the last
         //! `groups` groups of 256 queries run as `split` blocks of 256/split queries each, so the
         //! waves that start last are shorter (groups = 0: one block per group).
         void setTailSplit(unsigned int groups, unsigned int split)
@@ -274,6 +393,7 @@ class LBVHTraverser : public Tunable<unsigned int>
             if (split != 1 && split != 2 && split != 4) throw std::invalid_argument("the tail split must be 1, 2 or 4");
             m_tail_groups = groups;
             m_tail_split = split;
+            m_tail_set = true;
             }
         unsigned int getTailGroups() const { return m_tail_groups; }
         unsigned int getTailSplit() const { return m_tail_split; }
@@ -330,6 +450,24 @@ void LBVHTraverser::traverse(const LaunchParameters& params, const LBVH& lbvh, c
 
     const unsigned int* order = (m_order && m_order_n == query.size()) ? m_order : nullptr;
     const dim3 grid(div_up(query.size(), block));
+    constexpr bool reference = std::is_same<QueryOpT, SphereQueryOp>::value;
+    if constexpr (reference)
+        {
+        if (m_variant == TraversalVariant::Quantized)
+            {
+            launch_front(params, query, out, images, order, lbvh.getNNodes(),
+                         gpu::kernel::front::QuantizedSource{m_data.get(), float3(), float3(), float3(), lbvh.getNInternal()});
+            check_launch("lbvh_traverse");
+            return;
+            }
+        if (m_variant == TraversalVariant::FloatRope || m_variant == TraversalVariant::FloatRopeExact)
+            {
+            launch_front(params, query, out, images, order, lbvh.getNNodes(),
+                         gpu::kernel::front::RopeSource{m_float.get(), lbvh.getNInternal()});
+            check_launch("lbvh_traverse");
+            return;
+            }
+        }
     if (m_variant == TraversalVariant::Quantized)
         {
         hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_ropes<OutputOpT, QueryOpT, TranslateOpT>), grid, dim3(block), 0,

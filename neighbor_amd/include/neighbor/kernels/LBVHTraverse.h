@@ -467,11 +467,9 @@ template<class O>
 struct places_rows<O, typename std::enable_if<O::kPlacedRows>::type> : std::true_type {};
 
 template<class OutputOpT>
-__device__ __forceinline__ void place_rows(const OutputOpT& out, const unsigned int t, const unsigned int idx, const bool valid,
-                                           const unsigned int group = 0u, const unsigned int lead = 0u,
-                                           const unsigned int* order = nullptr, const unsigned int n = 0u)
+__device__ __forceinline__ void place_rows(const OutputOpT& out, const unsigned int t, const unsigned int idx, const bool valid)
     {
-    if constexpr (places_rows<OutputOpT>::value) out.place(t, idx, valid, group, lead, order, n);
+    if constexpr (places_rows<OutputOpT>::value) out.place(t, idx, valid);
     }
 
 struct Stage
@@ -1036,45 +1034,6 @@ __global__ void __launch_bounds__(256) lbvh_traverse_wave(const OutputOpT out,
     wave::walk<OutputOpT, QueryOpT, TranslateOpT, TransformOpT, STATS>(
         out, nodes, points, primitive, root_box, root, LBVHSentinel, query, images, transform, valid, idx, n_internal,
         n_nodes, stage, lds.wave_compact(), STATS ? visits + 3u * (t >> 6) : nullptr);
-    }
-
-//! lbvh_traverse_wave for the compacted exact counts and pair fills (wave::compactable ops),
-//! compiled for eight waves per SIMD: 64 VGPRs with a few spilled instead of 72 at seven waves
-//! (the fill of the N=10^6 exact step measured 0.74 against 0.78 ms).  The reference-query
-//! walks and the walks with a visit log keep the kernel above.  Blocks map to queries by
-//! wave::tail_block (tail_groups = 0: the plain XCD map).
-template<class OutputOpT, class QueryOpT, class TranslateOpT, class TransformOpT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8)))
-lbvh_traverse_wave_pairs(const OutputOpT out,
-                         const float4* __restrict__ nodes,
-                         const float4* __restrict__ points,
-                         const unsigned int* __restrict__ primitive,
-                         const float3* __restrict__ root_lo,
-                         const float3* __restrict__ root_hi,
-                         const int root,
-                         const QueryOpT query,
-                         const TranslateOpT images,
-                         const TransformOpT transform,
-                         const unsigned int* __restrict__ order,
-                         const unsigned int n_nodes,
-                         const unsigned int tail_groups,
-                         const unsigned int tail_split)
-    {
-    __shared__ StageStorage<OutputOpT, QueryOpT> lds;
-    const unsigned int n = query.size();
-    const wave::BlockSpan span = wave::tail_block(blockIdx.x, (n + 255u) / 256u, tail_groups, tail_split);
-    if (!span.live) return;
-    wave::Stage stage = lds.lane_stage();
-    const unsigned int lane = threadIdx.x & 63u;
-    const unsigned int t = span.first + (threadIdx.x >> 6) * span.per_wave + lane;
-    const unsigned int n_internal = (n_nodes - 1u) / 2u;
-    const bool valid = lane < span.per_wave && t < n;
-    const unsigned int idx = valid ? (order ? order[t] : t) : 0u;
-    const BoundingBox root_box(*root_lo, *root_hi);
-    wave::place_rows(out, t, idx, valid, span.first - span.lead, span.lead, order, n);
-    wave::walk<OutputOpT, QueryOpT, TranslateOpT, TransformOpT, false>(
-        out, nodes, points, primitive, root_box, root, LBVHSentinel, query, images, transform, valid, idx, n_internal,
-        n_nodes, stage, lds.wave_compact(), nullptr);
     }
 
 } // end namespace kernel

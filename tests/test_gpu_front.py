@@ -1,0 +1,192 @@
+"""The walk by node fronts (GPU) against the oracle: sizes around its groups, batches, buckets and
+launch rules, query orders, scattered and unusual queries, every traversal variant and output."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def nb():
+    import neighbor_amd
+    return neighbor_amd
+
+
+@pytest.fixture(scope="module")
+def orc():
+    import oracle
+    return oracle
+
+
+def host(t):
+    return t.cpu().numpy()
+
+
+def points_of(n, rng, kind):
+    L = max((n / 0.85) ** (1.0 / 3.0), 1.0)
+    p = rng.random((n, 3)).astype(np.float32) * np.float32(L)
+    if kind == "lattice":       # many equal distances and coordinates
+        p = np.round(p * 2) / np.float32(2)
+    if kind == "copies":        # runs of coincident points
+        p = p[rng.integers(0, max(n // 40, 1), n)]
+    return np.ascontiguousarray(p, np.float32), float(np.float32(L))
+
+
+# 16 / 32 / 64: group, run and wave; 2048: chunk; 16384, 32768, 65536: queries per team
+SIZES = [1, 2, 15, 16, 17, 32, 33, 63, 64, 65, 130, 1023, 1025, 2049, 16384, 16385, 32769, 65537]
+
+
+@pytest.mark.parametrize("kind", ["uniform", "lattice", "copies"])
+@pytest.mark.parametrize("n", SIZES)
+def test_reference_query(nb, orc, n, kind):
+    """Counts and lists of every variant equal the oracle's traversal, in order, for queries in
+    particle, Morton and random order, with and without images."""
+    import torch
+    from neighbor_amd.workloads import images27
+    if kind != "uniform" and n > 20000:
+        pytest.skip("large sizes with uniform points only")
+    rng = np.random.default_rng(n)
+    pts, L = points_of(n, rng, kind)
+    rad = 0.25 if kind == "copies" else None
+    r = 1.0 if kind == "copies" else 1.7
+    # the points themselves, some outside the box, some with other radii (zero, large, negative)
+    sph = np.concatenate([pts, np.full((n, 1), r, np.float32)], 1).astype(np.float32)
+    sph[::7, 3] = 0.0
+    if n <= 3000:
+        sph[3::11, 3] = 0.6 * L
+        sph[5::13, :3] += np.float32(1.5 * L)
+        sph[6::17, 3] = -r
+    tree = orc.build(pts, [0, 0, 0], [L] * 3, -1.0 if rad is None else rad)
+    records = orc.compress(tree)
+    lb = nb.LBVH()
+    lb.build(torch.from_numpy(pts).cuda(), [0, 0, 0], [L] * 3, radius=rad)
+    shuffled = rng.permutation(n).astype(np.int32)
+    d_sph = torch.from_numpy(sph).cuda()
+    images = images27(L) if n < 40000 else images27(L)[9:18]
+    for imgs in (images, None):
+        ref = orc.traverse(n, records, sph, imgs, triplets=True)
+        counts = ref["counts"].astype(np.int64)
+        most = int(counts.max()) if n else 0
+        for variant in (nb.NB_VARIANT_QUANTIZED, nb.NB_VARIANT_FLOAT_ROPE, nb.NB_VARIANT_WAVE_QUANTIZED):
+            tr = nb.LBVHTraverser(variant=variant)
+            tr.set_bucket_size(24)
+            tr.setup(lb)
+            d_img = None if imgs is None else torch.from_numpy(imgs).cuda()
+            for order in (None, lb.device_pointers()["primitive"], torch.from_numpy(shuffled).cuda()):
+                got = host(tr.count(lb, d_sph, images=d_img, order=order)).view(np.uint32)
+                assert np.array_equal(got, ref["counts"]), (variant, imgs is None)
+            cut = max(min(most, 40), 1)
+            lst, nn = tr.neighbor_list(lb, d_sph, cut, images=d_img)
+            assert np.array_equal(host(nn).view(np.uint32), ref["counts"])
+            pos = np.concatenate([[0], np.cumsum(counts)])[:-1]
+            want = np.zeros((n, cut), np.int64)
+            for k in range(cut):
+                have = counts > k
+                want[have, k] = ref["prim"][pos[have] + k]
+            assert np.array_equal(host(lst).astype(np.int64), want)
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("bucket", [1, 16, 33, 64])
+def test_exact_query(nb, orc, n, bucket):
+    """Exact counts and rows (image-major, then Morton order) equal the FP64 cell list."""
+    import torch
+    from neighbor_amd.api import exact_rows, exclusive_scan
+    from neighbor_amd.workloads import images27
+    if n > 2049 and bucket not in (16, 64):
+        pytest.skip("large sizes with two bucket sizes only")
+    rng = np.random.default_rng(n + 77)
+    pts, L = points_of(n, rng, "lattice" if n % 2 and n < 3000 else "uniform")
+    r = 1.5
+    sph = np.concatenate([pts, np.full((n, 1), r, np.float32)], 1).astype(np.float32)
+    ref = orc.exact_bruteforce(pts, sph, images27(L, dtype=np.float64)) if n < 3000 else orc.exact_celllist(pts, sph, [L] * 3, r)
+    d_pts, d_sph = torch.from_numpy(pts).cuda(), torch.from_numpy(sph).cuda()
+    d_img = torch.from_numpy(images27(L, dtype=np.float64)).cuda()
+    lb = nb.LBVH()
+    lb.build(d_pts, [0, 0, 0], [L] * 3)
+    tr = nb.LBVHTraverser(variant=nb.NB_VARIANT_WAVE)
+    tr.set_bucket_size(bucket)
+    tr.setup(lb)
+    counts = ref["counts"].astype(np.int64)
+    offs = np.concatenate([[0], np.cumsum(counts)])
+    for order in (None, lb.device_pointers()["primitive"], torch.from_numpy(rng.permutation(n).astype(np.int32)).cuda()):
+        got = tr.exact_count(lb, d_sph, d_pts, images=d_img, order=order)
+        assert np.array_equal(host(got).view(np.uint32), ref["counts"])
+        start = exclusive_scan(got)
+        neigh = torch.full((int(offs[-1]) + 1,), -1, dtype=torch.int32, device="cuda")
+        img = torch.full((int(offs[-1]) + 1,), 77, dtype=torch.uint8, device="cuda")
+        filled = exact_rows(tr, lb, d_sph, d_pts, start, got, neigh, img, images=d_img, order=order)
+        assert np.array_equal(host(filled).view(np.uint32), ref["counts"])
+        nj, nk = host(neigh)[:-1].astype(np.int64), host(img)[:-1].astype(np.int64)
+        assert int(neigh[-1]) == -1 and int(img[-1]) == 77
+        i = np.repeat(np.arange(n), counts)
+        assert np.array_equal(np.lexsort((nk, i)), np.arange(i.size)), "rows are not image by image"
+        a = np.lexsort((nj, nk, i))
+        b = np.lexsort((ref["j"], ref["k"], i))
+        assert np.array_equal(nk[a], ref["k"].astype(np.int64)[b]) and np.array_equal(nj[a], ref["j"].astype(np.int64)[b])
+
+
+@pytest.mark.parametrize("n", [40, 5000, 70000])
+def test_unusual_queries(nb, orc, n):
+    """Queries at infinity, NaN, and radii beyond the walk's range beside ordinary ones: the
+    ordinary rows are the oracle's, the others those of the definition."""
+    import torch
+    rng = np.random.default_rng(5)
+    pts, L = points_of(n, rng, "uniform")
+    sph = np.concatenate([pts, np.full((n, 1), 1.5, np.float32)], 1).astype(np.float32)
+    odd = rng.choice(n, 8, replace=False)
+    sph[odd[0], 0] = np.inf
+    sph[odd[1], 1] = np.nan
+    sph[odd[2], 3] = np.inf
+    sph[odd[3], 3] = 1e30
+    sph[odd[4], 3] = np.nan
+    sph[odd[5], :3] = 1e20
+    sph[odd[6], :3] = -3e38
+    sph[odd[7], 3] = 3e38
+    d_pts, d_sph = torch.from_numpy(pts).cuda(), torch.from_numpy(sph).cuda()
+    lb = nb.LBVH()
+    lb.build(d_pts, [0, 0, 0], [L] * 3)
+    ref = orc.traverse(n, orc.compress(orc.build(pts, [0, 0, 0], [L] * 3)), sph, None)["counts"]
+    for variant in (nb.NB_VARIANT_QUANTIZED, nb.NB_VARIANT_FLOAT_ROPE, nb.NB_VARIANT_WAVE_QUANTIZED):
+        tr = nb.LBVHTraverser(variant=variant)
+        tr.setup(lb)
+        assert np.array_equal(host(tr.count(lb, d_sph)).view(np.uint32), ref)
+    tr = nb.LBVHTraverser(variant=nb.NB_VARIANT_WAVE)
+    tr.setup(lb)
+    got = host(tr.exact_count(lb, d_sph, d_pts)).astype(np.int64)
+    plain = np.setdiff1d(np.arange(n), odd)
+    check = np.concatenate([plain[:: max(1, plain.size // 400)], odd])
+    with np.errstate(all="ignore"):
+        for q in check:
+            d = sph[q, :3].astype(np.float64) - pts.astype(np.float64)
+            d2 = (d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1]) + d[:, 2] * d[:, 2]
+            want = int((d2 <= np.float64(sph[q, 3]) * np.float64(sph[q, 3])).sum())
+            assert got[q] == want, (q, sph[q])
+
+
+def test_two_streams_share_a_traverser(nb, orc):
+    """Unordered queries (sorted on the device in the traverser's workspaces) on two streams and
+    with other numbers of queries in turn."""
+    import torch
+    rng = np.random.default_rng(9)
+    pts, L = points_of(30000, rng, "uniform")
+    lb = nb.LBVH()
+    lb.build(torch.from_numpy(pts).cuda(), [0, 0, 0], [L] * 3)
+    tr = nb.LBVHTraverser()
+    tr.setup(lb)
+    records = orc.compress(orc.build(pts, [0, 0, 0], [L] * 3))
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(6)]
+    sets, outs = [], []
+    for i in range(12):
+        sph = np.concatenate([rng.random((2000 + 3001 * (i % 4), 3)) * L, np.full((2000 + 3001 * (i % 4), 1), 1.6)], 1).astype(np.float32)
+        sets.append((sph, torch.from_numpy(sph).cuda()))
+    torch.cuda.synchronize()
+    for i, (_, d) in enumerate(sets):
+        with torch.cuda.stream(streams[i % 6]):
+            outs.append(tr.count(lb, d, stream=streams[i % 6]))
+    torch.cuda.synchronize()
+    for (sph, _), out in zip(sets, outs):
+        assert np.array_equal(host(out).view(np.uint32), orc.traverse(30000, records, sph, None)["counts"])
