@@ -301,14 +301,14 @@ int nb_lbvh_set_span_lds_limit(nb_lbvh* lbvh, uint32_t limit);
 
 /* ------------------------------------------------------------------ batched boxes
  * (No reference counterpart.)  Many independent boxes built as one forest with one sort and
- * traversed by one persistent launch: points of all boxes concatenated (box b holds
+ * traversed by one launch: points of all boxes concatenated (box b holds
  * [offsets[b], offsets[b+1])), each box with its own lower/upper corner (its periodic cell).
  * Queries are the points themselves: spheres (device, N x float4 x, y, z, r) in the same
  * order, each queried against its own box only (27 images of the box when periodic != 0).
  * Outputs are indexed by the global point index and neighbors are global indices.  The
  * pair semantics are those of nb_traverse_exact_pairs. */
 typedef struct nb_batch nb_batch;
-#define NB_BATCH_WAVE 0   /* one rope path per wave of 64 Morton-consecutive queries */
+#define NB_BATCH_WAVE 0   /* one walk by node fronts per wave of 64 Morton-consecutive queries */
 #define NB_BATCH_LANE 1   /* one rope path per lane */
 int nb_batch_create(nb_batch** out);
 int nb_batch_destroy(nb_batch* batch);
@@ -317,8 +317,8 @@ int nb_batch_destroy(nb_batch* batch);
 int nb_batch_build(nb_batch* batch, const float* points, uint32_t N, const uint32_t* offsets, const float* box_lo,
                    const float* box_hi, uint32_t nbox, void* stream);
 /* Tunables: block (hierarchy kernel, multiple of 32 in [32, 1024]), bucket (leaves per bucket,
- * 1..64), variant (NB_BATCH_*), grid (persistent blocks, 0 = 8 per CU).  Bucket changes take
- * effect at nb_batch_setup. */
+ * 1..64), variant (NB_BATCH_*), grid (blocks of the traversal, 0 = one wave per 64 queries of a
+ * box).  Bucket changes take effect at nb_batch_setup. */
 int nb_batch_set_params(nb_batch* batch, uint32_t block, uint32_t bucket, int variant, uint32_t grid);
 int nb_batch_get_params(const nb_batch* batch, uint32_t* block, uint32_t* bucket, int* variant, uint32_t* grid);
 /* Bucket records of the built forest (after every build). */

@@ -1,4 +1,4 @@
-"""Batched boxes over the C ABI: one forest build, one persistent traversal, one graph.
+"""Batched boxes over the C ABI: one forest build, one traversal launch, one graph.
 
 Points of all boxes are concatenated (box b holds rows offsets[b]:offsets[b+1]); each box
 has its own lower/upper corner (its periodic cell).  Queries are the points themselves,

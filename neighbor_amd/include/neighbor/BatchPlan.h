@@ -145,7 +145,6 @@ class BatchPlan
                 // eager run first: every allocation happens here, outside the capture
                 step();
                 NEIGHBOR_HIP_CHECK(hipStreamSynchronize(m_stream));
-                batch.setGrid(batch.gridSize());
                 NEIGHBOR_HIP_CHECK(hipStreamBeginCapture(m_stream, hipStreamCaptureModeRelaxed));
                 step();
                 NEIGHBOR_HIP_CHECK(hipStreamEndCapture(m_stream, &m_graph));

@@ -5,7 +5,7 @@
 // the single-tree pipeline once over all boxes with 64-bit (box, Morton code) keys
 // (kernels/Batch.h), so every box is a subtree shaped like its own tree, and finds the
 // box roots and the 64-query work items.  setupTraversal() writes the bucket records;
-// traverse() runs one persistent launch over all items with any output op (count, pair
+// traverse() runs one launch over all items with any output op (count, pair
 // list, rows).  Queries are the points themselves (one sphere per point), each against
 // its own box, with the 27 periodic images of that box.  Every launch is on one stream
 // with no host synchronization, so the whole sequence can be captured in a graph.
@@ -150,7 +150,7 @@ class LBVHBatch
             check_launch("batch records");
             }
 
-        //! One persistent launch over all items.  spheres: one float4 (x, y, z, r) per point
+        //! One launch over all items.  spheres: one float4 (x, y, z, r) per point
         //! (original order); the output op is indexed by the original point index.
         template<class OutputOpT>
         void traverse(const OutputOpT& out, const float4* spheres, bool periodic, BatchVariant variant, hipStream_t stream)
@@ -158,25 +158,18 @@ class LBVHBatch
             if (m_N == 0) return;
             if (m_records.size() == 0) throw std::runtime_error("setupTraversal() first");
             const ExactSphereQueryOp query(spheres, m_N, m_points);
-            hipLaunchKernelGGL(gpu::radix::kernel::fill_zero, dim3(1), dim3(64), 0, stream, m_counters.get(),
-                               static_cast<size_t>(gpu::batch::kQueues));
             const unsigned long long* n_items = m_item_offsets.get() + m_nbox;
             const unsigned int grid = gridSize();
             if (variant == BatchVariant::Lane)
                 hipLaunchKernelGGL((gpu::batch::kernel::batch_traverse<true, OutputOpT, ExactSphereQueryOp>), dim3(grid), dim3(256), 0,
                                    stream, out, m_records.get(), m_sorted.get(), m_indexes.current().get(), m_lo.get(), m_hi.get(),
                                    m_rope.get(), m_roots.get(), m_offsets, m_box_lo, m_box_hi, m_items.get(), n_items,
-                                   m_counters.get(), query, periodic ? 1u : 0u, m_N + m_Ni);
-            else if constexpr (gpu::kernel::wave::compactable<OutputOpT, ExactSphereQueryOp>::value)
-                hipLaunchKernelGGL((gpu::batch::kernel::batch_traverse_pairs<OutputOpT, ExactSphereQueryOp>), dim3(grid), dim3(256),
-                                   0, stream, out, m_records.get(), m_sorted.get(), m_indexes.current().get(), m_lo.get(),
-                                   m_hi.get(), m_rope.get(), m_roots.get(), m_offsets, m_box_lo, m_box_hi, m_items.get(), n_items,
-                                   m_counters.get(), query, periodic ? 1u : 0u, m_N + m_Ni);
+                                   query, periodic ? 1u : 0u, m_N + m_Ni);
             else
                 hipLaunchKernelGGL((gpu::batch::kernel::batch_traverse<false, OutputOpT, ExactSphereQueryOp>), dim3(grid), dim3(256), 0,
                                    stream, out, m_records.get(), m_sorted.get(), m_indexes.current().get(), m_lo.get(), m_hi.get(),
                                    m_rope.get(), m_roots.get(), m_offsets, m_box_lo, m_box_hi, m_items.get(), n_items,
-                                   m_counters.get(), query, periodic ? 1u : 0u, m_N + m_Ni);
+                                   query, periodic ? 1u : 0u, m_N + m_Ni);
             check_launch("batch_traverse");
             }
 
@@ -204,7 +197,7 @@ class LBVHBatch
             m_bucket = bucket;
             }
         unsigned int getBucket() const { return m_bucket; }
-        //! Blocks of the persistent traversal (0: from the device's CU count).
+        //! Blocks of the traversal (0: one wave per work item).
         void setGrid(unsigned int g) { m_grid = g; }
 
         unsigned int getN() const { return m_N; }
@@ -243,7 +236,7 @@ class LBVHBatch
         shared_array<float4> m_sorted, m_records;
         buffered_array<unsigned long long> m_keys;
         buffered_array<unsigned int> m_indexes;
-        shared_array<unsigned int> m_work, m_item_counts, m_counters, m_code_one;
+        shared_array<unsigned int> m_work, m_item_counts, m_code_one;
         shared_array<unsigned long long> m_item_offsets;
         shared_array<gpu::batch::Item> m_items;
         shared_array<unsigned char> m_scan_scratch;
@@ -257,15 +250,12 @@ class LBVHBatch
             }
 
     public:
-        //! Blocks of the persistent traversal: the set value, else 8 per CU.
+        //! Blocks of the traversal (four waves each): the set value, else one wave per work item,
+        //! at most N / 64 items and one more per box.
         unsigned int gridSize() const
             {
             if (m_grid) return m_grid;
-            int dev = 0, cus = 0;
-            NEIGHBOR_HIP_CHECK(hipGetDevice(&dev));
-            NEIGHBOR_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-            // enough 256-thread blocks to fill every CU; waves leave when the items run out
-            return static_cast<unsigned int>(std::max(cus, 1)) * 8u;
+            return div_up(m_N / gpu::batch::kItemQueries + m_nbox + 1u, 4u);
             }
 
     private:
@@ -354,10 +344,9 @@ class LBVHBatch
                 grew = true;
                 shared_array<gpu::batch::Item>(max_items, dev).swap(m_items);
                 }
-            if (m_counters.size() == 0)
+            if (m_code_one.size() == 0)
                 {
                 grew = true;
-                shared_array<unsigned int>(gpu::batch::kQueues, dev).swap(m_counters);
                 shared_array<unsigned int>(1, dev).swap(m_code_one);
                 }
             if (grew) ++*m_generation;

@@ -10,13 +10,13 @@
 //   (bubble)         the single-tree bubble kernels, unchanged;
 //   batch_roots      the subtree root of every box;
 //   batch_items      work items of up to 64 consecutive (Morton-ordered) queries of one box.
-// Traversal: persistent kernels claim items from eight queues, one per XCD, each a
-// contiguous range of items (so one XCD's L2 holds a few boxes at a time) and steal from
-// the other queues when their own is empty.  Queries are the points themselves; the walk
+// Traversal: one wave per item, each XCD a contiguous range of items (so its L2 holds a few
+// boxes at a time).  Queries are the points themselves; the walk
 // of an item covers its box's subtree only, with the box's own periodic images.
 #ifndef NEIGHBOR_KERNELS_BATCH_H_
 #define NEIGHBOR_KERNELS_BATCH_H_
 
+#include "FrontWalk.h"
 #include "LBVHBuild.h"
 #include "LBVHTraverse.h"
 
@@ -33,7 +33,6 @@ namespace walk_kernels = ::neighbor::gpu::kernel;
 
 constexpr unsigned int kCodeBits = 30;
 constexpr unsigned int kItemQueries = 64;      //!< queries per work item (one wave)
-constexpr unsigned int kQueues = walk_kernels::wave::kXcds;  //!< item queues, one per XCD
 
 //! Box of global point i: the last b with offsets[b] <= i (offsets has nbox + 1 entries).
 __device__ __forceinline__ unsigned int box_of(const uint32_t* __restrict__ offsets, unsigned int nbox, uint32_t i)
@@ -196,24 +195,16 @@ __global__ void __launch_bounds__(256) batch_items(const uint32_t* __restrict__ 
     for (uint32_t f = 0; f < n; f += kItemQueries, ++t) items[t] = Item{b, f};
     }
 
-//! Claim the next item for this wave from queue `q` (wave-uniform result).
-__device__ __forceinline__ unsigned long long claim(unsigned int* __restrict__ counters, unsigned int q)
-    {
-    unsigned int v = 0;
-    if ((threadIdx.x & 63u) == 0u) v = atomicAdd(&counters[q], 1u);
-    return __builtin_amdgcn_readfirstlane(v);
-    }
-
-//! Items [begin, end) of queue q out of n items.
-__device__ __forceinline__ void queue_range(unsigned long long n, unsigned int q, unsigned long long& begin,
-                                            unsigned long long& end)
-    {
-    begin = n * q / kQueues;
-    end = n * (q + 1u) / kQueues;
-    }
-
-//! Persistent traversal of the forest.  LANE_WALK: each lane walks its own rope path
-//! (bucket records, leaves tested one by one); otherwise wave::walk.
+//! Traversal of the forest, an item per wave and turn.  Waves take items in a fixed order: block b
+//! serves the items of the contiguous range of its XCD (b % 8), so an XCD's L2 holds a few boxes at
+//! a time, and with the default grid every wave has one item and the dispatcher balances them.
+//! (Claiming items from eight queues cost an atomic on the queues' one cache line per item and
+//! eight more per wave at the end, one after the other: the step below took 3689 instead of 2454 us.)
+//!  LANE_WALK: each lane walks its own rope path
+//! (bucket records, leaves tested one by one); otherwise each wave's item by node fronts
+//! (front::walk): a box's up to 27 images start together, where a rope walk took one after the
+//! other.  512 boxes of 256 to 16384 points (2*10^6 points, 27 images, 32 leaves per bucket):
+//! build, count, scan and fill 3913 us with rope walks from the queues, 2454 us so.
 template<bool LANE_WALK, class OutputOpT, class QueryOpT>
 __device__ __forceinline__ void batch_traverse_body(const OutputOpT& out,
                                                     const float4* __restrict__ nodes,
@@ -228,28 +219,24 @@ __device__ __forceinline__ void batch_traverse_body(const OutputOpT& out,
                                                     const float3* __restrict__ box_hi,
                                                     const Item* __restrict__ items,
                                                     const unsigned long long* __restrict__ n_items_ptr,
-                                                    unsigned int* __restrict__ counters,
                                                     const QueryOpT& query,
                                                     const unsigned int periodic,
                                                     const unsigned int n_nodes)
     {
-    // the lane walk writes its hits directly: no staging storage
-    __shared__ walk_kernels::StageStorage<typename std::conditional<LANE_WALK, int, OutputOpT>::type, QueryOpT> lds;
-    walk_kernels::wave::Stage stage = lds.lane_stage();
+    namespace front = walk_kernels::front;
+    typedef front::BucketSource<NullTransformOp> Source;
+    constexpr size_t kPart = LANE_WALK ? 16 : front::FrontLds<OutputOpT>::kPart;
+    __shared__ alignas(16) unsigned char lds[4][kPart];
+    const unsigned int wid = static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)));
     const unsigned int lane = threadIdx.x & 63u;
     const unsigned int n_internal = (n_nodes - 1u) / 2u;
     const unsigned long long n_items = *n_items_ptr;
-    const unsigned int home = blockIdx.x % kQueues;
-
-    for (unsigned int qi = 0; qi < kQueues; ++qi)
+    const unsigned long long n_blocks = (n_items + 3ull) / 4ull;
+    for (unsigned long long turn = blockIdx.x; turn < n_blocks; turn += gridDim.x)
         {
-        const unsigned int q = (home + qi) % kQueues;
-        unsigned long long begin, end;
-        queue_range(n_items, q, begin, end);
-        for (;;)
+        const unsigned long long t = 4ull * walk_kernels::wave::xcd_block(static_cast<unsigned int>(turn), static_cast<unsigned int>(n_blocks)) + wid;
+        if (t < n_items)
             {
-            const unsigned long long t = begin + claim(counters, q);
-            if (t >= end) break;
             const Item it = items[t];
             const uint32_t s = offsets[it.box];
             const uint32_t nb = offsets[it.box + 1] - s;
@@ -315,8 +302,14 @@ __device__ __forceinline__ void batch_traverse_body(const OutputOpT& out,
                 }
             else
                 {
-                walk_kernels::wave::walk(out, nodes, points, primitive, root_box, root, stop, query, images, NullTransformOp(), valid, idx,
-                           n_internal, n_nodes, stage, lds.wave_compact());
+                const float4 qd = valid ? query.setup(idx) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                const Source src{nodes, points, primitive, NullTransformOp(), n_internal};
+                front::FrontWave& W = *reinterpret_cast<front::FrontWave*>(lds[wid]);
+                front::FrontPairs& P = *reinterpret_cast<front::FrontPairs*>(lds[wid] + sizeof(front::FrontWave));
+                const bool walked = !rooted || (front::takes<QueryOpT>(valid, qd, images, root_box)
+                    && front::walk<false>(out, src, root, root_box, query, images, valid, idx, qd, 2u * nb - 1u, W, P, nullptr));
+                if (valid && !rooted) out.finalize(out.setup(idx, qd));
+                else if (valid && !walked) front::lane_walk(out, src, root, stop, root_box, query, images, idx, qd, n_nodes);
                 }
             }
         }
@@ -328,24 +321,15 @@ __device__ __forceinline__ void batch_traverse_body(const OutputOpT& out,
         const float3* __restrict__ tree_hi, const int* __restrict__ rope, const int* __restrict__ roots,          \
         const uint32_t* __restrict__ offsets, const float3* __restrict__ box_lo, const float3* __restrict__ box_hi, \
         const Item* __restrict__ items, const unsigned long long* __restrict__ n_items_ptr,                       \
-        unsigned int* __restrict__ counters, const QueryOpT query, const unsigned int periodic, const unsigned int n_nodes
+        const QueryOpT query, const unsigned int periodic, const unsigned int n_nodes
 #define NEIGHBOR_BATCH_TRAVERSE_ARGS                                                                              \
-    out, nodes, points, primitive, tree_lo, tree_hi, rope, roots, offsets, box_lo, box_hi, items, n_items_ptr, counters, \
+    out, nodes, points, primitive, tree_lo, tree_hi, rope, roots, offsets, box_lo, box_hi, items, n_items_ptr, \
         query, periodic, n_nodes
 
 template<bool LANE_WALK, class OutputOpT, class QueryOpT>
-__global__ void __launch_bounds__(256) batch_traverse(NEIGHBOR_BATCH_TRAVERSE_PARAMS)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) batch_traverse(NEIGHBOR_BATCH_TRAVERSE_PARAMS)
     {
     batch_traverse_body<LANE_WALK, OutputOpT, QueryOpT>(NEIGHBOR_BATCH_TRAVERSE_ARGS);
-    }
-
-//! batch_traverse of the wave walk for the compacted exact pair fills, compiled for eight
-//! waves per SIMD as the single-tree pair fill is (lbvh_traverse_wave_pairs).
-template<class OutputOpT, class QueryOpT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8)))
-batch_traverse_pairs(NEIGHBOR_BATCH_TRAVERSE_PARAMS)
-    {
-    batch_traverse_body<false, OutputOpT, QueryOpT>(NEIGHBOR_BATCH_TRAVERSE_ARGS);
     }
 
 #undef NEIGHBOR_BATCH_TRAVERSE_PARAMS

@@ -514,8 +514,8 @@ __device__ __forceinline__ void write_hits(unsigned int* __restrict__ neigh, uns
         }
     }
 
-//! The walk over the subtree of `root` for one query per lane, by one wave or, TEAM, by the four
-//! waves of a block for the same queries.
+//! The walk over the subtree of `root` (n_nodes nodes) for one query per lane, by one wave or, TEAM,
+//! by the four waves of a block for the same queries; false: not walked (queries too scattered).
 /*!
  * Front: a stack of (node, image) entries, the first of the traversal order on top.  A step
  * takes up to 64 entries off the top, tests them, and puts the children of the inner nodes
@@ -612,7 +612,7 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
             W.hi[lane >> 4] = make_float4(ghi.x, ghi.y, ghi.z, 0.0f);
             }
         // side of the cube that holds one of the tree's leaves on average
-        const float leaves = static_cast<float>(n_internal + 1u);
+        const float leaves = 0.5f * static_cast<float>(n_nodes + 1u);
         const float cell = exp2f(log2f(fmaxf(root_box.hi.x - root_box.lo.x, 0.0f) * fmaxf(root_box.hi.y - root_box.lo.y, 0.0f)
                                        * fmaxf(root_box.hi.z - root_box.lo.z, 0.0f) / leaves) * (1.0f / 3.0f));
         const auto wider = [](const float3& a, const float3& b, const float side) {

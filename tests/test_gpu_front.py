@@ -190,3 +190,34 @@ def test_two_streams_share_a_traverser(nb, orc):
     torch.cuda.synchronize()
     for (sph, _), out in zip(sets, outs):
         assert np.array_equal(host(out).view(np.uint32), orc.traverse(30000, records, sph, None)["counts"])
+
+
+@pytest.mark.parametrize("grid", [0, 1, 3, 500])
+def test_batch_grids(nb, orc, grid):
+    """Boxes of sizes around a wave's 64 queries, by grids of fewer and of more waves than items."""
+    import torch
+    from neighbor_amd.batch import LBVHBatch
+    from neighbor_amd.workloads import batched_boxes, images27, spheres_from_points
+    sizes = [1, 2, 63, 64, 65, 128, 129, 700, 3, 2049]
+    pts, offsets, lo, hi = batched_boxes(sizes=sizes, seed=3)
+    r = 1.2
+    sph = spheres_from_points(pts, r)
+    b = LBVHBatch()
+    b.set_params(bucket=16, grid=grid)
+    b.build(torch.from_numpy(pts).cuda(), torch.from_numpy(offsets.astype(np.int32)).cuda(), torch.from_numpy(lo).cuda(),
+            torch.from_numpy(hi).cuda())
+    b.setup()
+    d_sph = torch.from_numpy(sph).cuda()
+    counts = host(b.count(d_sph)).astype(np.int64)
+    offs = np.concatenate([[0], np.cumsum(counts)])
+    neigh, image = b.pairs(d_sph, torch.from_numpy(offs).cuda(), total=int(offs[-1]))
+    nj, nk = host(neigh).astype(np.int64), host(image).astype(np.int64)
+    for k in range(len(sizes)):
+        s, e = int(offsets[k]), int(offsets[k + 1])
+        ref = orc.exact_bruteforce(pts[s:e], sph[s:e], images27(hi[k], dtype=np.float64))
+        assert np.array_equal(counts[s:e], ref["counts"].astype(np.int64))
+        i = np.repeat(np.arange(e - s), counts[s:e])
+        rows = slice(int(offs[s]), int(offs[e]))
+        a = np.lexsort((nj[rows], nk[rows], i))
+        c = np.lexsort((ref["j"], ref["k"], i))
+        assert np.array_equal(nk[rows][a], ref["k"].astype(np.int64)[c]) and np.array_equal(nj[rows][a] - s, ref["j"].astype(np.int64)[c])
