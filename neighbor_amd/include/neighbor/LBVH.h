@@ -289,26 +289,45 @@ void LBVH::build(const LaunchParameters& params, const InsertOpT& insert, const 
         m_header_dirty = false;
         }
 
-    // one block per 1024 primitives up to 2048 blocks: each folds its histogram into one of
-    // the eight copies (radix::kHistParts) with 256 atomics per pass (at 10^6 primitives 10.9 us
-    // at 2048 per block, 9.2 at 1024, 16 at 4096; one shared copy: 18.3 us, slower with more
-    // blocks)
-    const unsigned int code_blocks = std::min<unsigned int>(div_up(m_N, 1024), 2048u);
-    hipLaunchKernelGGL(gpu::kernel::lbvh_codes<InsertOpT>, dim3(code_blocks), dim3(256), 0, stream,
-                       insert, lo, hi, m_N, m_codes.current().get(), ws.hist, ws.passes, clear_begin, clear_words);
-    check_launch("lbvh_codes");
-
-    const bool alt = gpu::radix::sort_passes(m_codes.current().get(), m_indexes.current().get(),
-                                             m_codes.alternate().get(), m_indexes.alternate().get(),
-                                             m_N, true, ws, stream);
-    if (alt)
+    constexpr bool kGather = gpu::detail::point_leaves<InsertOpT>::value;
+    if (m_N <= gpu::kernel::kSmallTree)
         {
-        m_codes.flip();
-        m_indexes.flip();
+        // one chunk: everything in one workgroup and launch
+        hipLaunchKernelGGL(gpu::kernel::lbvh_small_build<InsertOpT>, dim3(1), dim3(gpu::radix::kernel::kSmallBlock), 0, stream,
+                           mutable_data(), insert, lo, hi, m_N, m_codes.current().get(), ws.passes, clear_begin, clear_words);
+        check_launch("lbvh_small_build");
+        recordSorted(stream);
+        return;
+        }
+    if (m_N <= gpu::radix::kernel::kRankSort)
+        {
+        // codes and places in one launch
+        hipLaunchKernelGGL(gpu::kernel::lbvh_ranked_codes<InsertOpT>, dim3(div_up(m_N, 64)), dim3(gpu::radix::kernel::kRankBlock), 0, stream,
+                           insert, lo, hi, m_N, m_codes.current().get(), m_indexes.current().get(), clear_begin, clear_words);
+        check_launch("lbvh_ranked_codes");
+        }
+    else
+        {
+        // one block per 1024 primitives up to 2048 blocks: each folds its histogram into one of
+        // the eight copies (radix::kHistParts) with 256 atomics per pass (at 10^6 primitives 10.9 us
+        // at 2048 per block, 9.2 at 1024, 16 at 4096; one shared copy: 18.3 us, slower with more
+        // blocks)
+        const unsigned int code_blocks = std::min<unsigned int>(div_up(m_N, 1024), 2048u);
+        hipLaunchKernelGGL(gpu::kernel::lbvh_codes<InsertOpT>, dim3(code_blocks), dim3(256), 0, stream,
+                           insert, lo, hi, m_N, m_codes.current().get(), ws.hist, ws.passes, clear_begin, clear_words);
+        check_launch("lbvh_codes");
+
+        const bool alt = gpu::radix::sort_passes(m_codes.current().get(), m_indexes.current().get(),
+                                                 m_codes.alternate().get(), m_indexes.alternate().get(),
+                                                 m_N, true, ws, stream);
+        if (alt)
+            {
+            m_codes.flip();
+            m_indexes.flip();
+            }
         }
 
     // point leaves: the hierarchy kernel also gathers each primitive's point into Morton order
-    constexpr bool kGather = gpu::detail::point_leaves<InsertOpT>::value;
     LBVHData tree = mutable_data();
     if constexpr (kGather)
         hipLaunchKernelGGL(gpu::kernel::lbvh_hierarchy<gpu::kernel::SortedPointGather<InsertOpT>>, dim3(div_up(m_N, block)),

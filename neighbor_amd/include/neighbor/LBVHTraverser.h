@@ -31,6 +31,7 @@
 
 #include <algorithm>
 #include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <type_traits>
 #include <vector>
@@ -203,16 +204,26 @@ class LBVHTraverser : public Tunable<unsigned int>
             stream_t stream = nullptr;
             std::shared_ptr<void> done;     //!< hipEvent_t
             };
-        //! Bounded: a launch finds its stream's workspace, a free one, or waits for the oldest.
-        static constexpr size_t kQuerySorts = 4;
-        std::vector<QuerySort> m_sorts;
-        size_t m_oldest_sort = 0;
+        //! Bounded: a launch finds its stream's workspace, a free one, or waits for the oldest.  The
+        //! lock is held from the sort to the record of `done` (several threads may traverse at
+        //! once); a copy of the traverser starts with none.
+        struct QuerySorts
+            {
+            static constexpr size_t kMost = 4;
+            std::vector<QuerySort> all;
+            size_t oldest = 0;
+            std::mutex lock;
+
+            QuerySorts() = default;
+            QuerySorts(const QuerySorts&) {}
+            QuerySorts& operator=(const QuerySorts&) { return *this; }
+            } m_sorts;
 
         QuerySort& query_sort(stream_t stream)
             {
-            for (QuerySort& s : m_sorts)
+            for (QuerySort& s : m_sorts.all)
                 if (s.stream == stream) return s;
-            for (QuerySort& s : m_sorts)
+            for (QuerySort& s : m_sorts.all)
                 {
                 if (hipEventQuery(static_cast<hipEvent_t>(s.done.get())) == hipSuccess)
                     {
@@ -221,17 +232,17 @@ class LBVHTraverser : public Tunable<unsigned int>
                     }
                 (void)hipGetLastError();    // not ready
                 }
-            if (m_sorts.size() < kQuerySorts)
+            if (m_sorts.all.size() < QuerySorts::kMost)
                 {
                 hipEvent_t e;
                 NEIGHBOR_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
                 QuerySort s;
                 s.done = std::shared_ptr<void>(static_cast<void*>(e), [](void* p) { (void)hipEventDestroy(static_cast<hipEvent_t>(p)); });
                 s.stream = stream;
-                m_sorts.push_back(s);
-                return m_sorts.back();
+                m_sorts.all.push_back(s);
+                return m_sorts.all.back();
                 }
-            QuerySort& s = m_sorts[m_oldest_sort++ % kQuerySorts];
+            QuerySort& s = m_sorts.all[m_sorts.oldest++ % QuerySorts::kMost];
             NEIGHBOR_HIP_CHECK(hipStreamWaitEvent(stream, static_cast<hipEvent_t>(s.done.get()), 0));
             s.stream = stream;
             return s;
@@ -249,6 +260,13 @@ class LBVHTraverser : public Tunable<unsigned int>
         const unsigned int* sorted_queries(QuerySort& s, const float4* spheres, const unsigned int n, stream_t stream)
             {
             const unsigned int bits = n <= (1u << 20) ? 16u : 24u;
+            if (n <= gpu::radix::kernel::kRankSort)
+                {
+                if (n > s.vals[0].size()) shared_array<unsigned int>(n, MemoryKind::Device).swap(s.vals[0]);
+                hipLaunchKernelGGL(gpu::kernel::query_order_ranked, dim3(div_up(n, 64)), dim3(gpu::radix::kernel::kRankBlock), 0, stream,
+                                   spheres, n, m_lbvh_lo.get(), m_lbvh_hi.get(), bits, s.vals[0].get());
+                return s.vals[0].get();
+                }
             const size_t words = gpu::radix::Workspace::words(n, bits);
             if (n > s.keys[0].size())
                 for (int i = 0; i < 2; ++i)
@@ -274,15 +292,17 @@ class LBVHTraverser : public Tunable<unsigned int>
             {
             constexpr bool placed = gpu::kernel::wave::places_rows<OutputOpT>::value;    // whole groups per block
             // queries in no given order are sorted first: a wave's queries must lie close together
-            QuerySort* sorted = nullptr;
             if constexpr (!placed)
                 if (!order && query.size() > kSortQueries && !capturing(params.stream))
                     {
-                    sorted = &query_sort(params.stream);
-                    order = sorted_queries(*sorted, query.spheres, query.size(), params.stream);
+                    const std::lock_guard<std::mutex> guard(m_sorts.lock);
+                    QuerySort& sort = query_sort(params.stream);
+                    launch_front_in_order(params, query, out, images, sorted_queries(sort, query.spheres, query.size(), params.stream),
+                                          n_nodes, src);
+                    NEIGHBOR_HIP_CHECK(hipEventRecord(static_cast<hipEvent_t>(sort.done.get()), params.stream));
+                    return;
                     }
             launch_front_in_order(params, query, out, images, order, n_nodes, src);
-            if (sorted) NEIGHBOR_HIP_CHECK(hipEventRecord(static_cast<hipEvent_t>(sorted->done.get()), params.stream));
             }
 
         template<class QueryOpT, class OutputOpT, class TranslateOpT, class SourceT>
@@ -354,11 +374,11 @@ class LBVHTraverser : public Tunable<unsigned int>
             }
 
         unsigned int m_bucket = 16;
-        //! Queries given without an order above which they are sorted first: the sort takes about
-        //! 40 us for few queries and 70 us for 10^6; a count of 1000 queries in random order (27
-        //! images) takes 89 us against 43 in Morton order, of 8000 179 against 71, and of 10^6
-        //! (one rope path per lane) 8.2 ms against 0.64.
-        static constexpr unsigned int kSortQueries = 1024;
+        //! Queries given without an order above which they are sorted first.  The sort takes about
+        //! 10 us for few queries and 70 us for 10^6.  Counts in random order and sorted here, with 27
+        //! images: 256 queries 44 us and 44, 512 71 and 54, 1000 89 and 44; without images 14 and 24,
+        //! 21 and 30, 34 and 33; 10^6 (one rope path per lane) 8.2 ms and 0.7.
+        static constexpr unsigned int kSortQueries = 256;
         //! Queries up to which four waves serve 64, 32 or 16 queries together: one wave's chain of
         //! steps takes longer than the chip needs for all of them.  Exact count and fill of 10,000
         //! points (27 images): 82 and 115 us with a wave per 64 queries, 48 and 61 with teams for

@@ -1155,6 +1155,25 @@ struct FrontLds
     };
 } // end namespace front
 
+//! Morton code (its first `bits` bits) of a query's center in the tree's root box.
+struct QueryCode
+    {
+    const float4* spheres;
+    float3 lo, L;
+    unsigned int bits;
+
+    __device__ __forceinline__ uint32_t operator()(const uint32_t i) const
+        {
+        const float4 c = spheres[i];
+        return morton3(fraction_to_bin((c.x - lo.x) / L.x), fraction_to_bin((c.y - lo.y) / L.y), fraction_to_bin((c.z - lo.z) / L.z)) >> (30u - bits);
+        }
+    };
+__device__ __forceinline__ QueryCode query_code(const float4* spheres, const float3* root_lo, const float3* root_hi, const unsigned int bits)
+    {
+    const float3 lo = *root_lo, hi = *root_hi;
+    return {spheres, lo, make_float3(hi.x - lo.x, hi.y - lo.y, hi.z - lo.z), bits};
+    }
+
 //! Morton codes of query centers in the tree's root box, their digit histograms, and the clearing
 //! of the sort's status words: the order in which a launch serves queries given without one.
 __global__ void __launch_bounds__(256) query_codes(const float4* __restrict__ spheres, const uint32_t n,
@@ -1165,15 +1184,12 @@ __global__ void __launch_bounds__(256) query_codes(const float4* __restrict__ sp
     __shared__ uint32_t s_hist[4 * radix::kRadix];
     for (unsigned int j = threadIdx.x; j < passes * radix::kRadix; j += blockDim.x) s_hist[j] = 0u;
     __syncthreads();
-    const float3 lo = *root_lo, hi = *root_hi;
-    const float3 L = make_float3(hi.x - lo.x, hi.y - lo.y, hi.z - lo.z);
+    const QueryCode code_of = query_code(spheres, root_lo, root_hi, bits);
     const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
     const size_t first = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     for (size_t i = first; i < n; i += stride)
         {
-        const float4 c = spheres[i];
-        const uint32_t code = morton3(fraction_to_bin((c.x - lo.x) / L.x), fraction_to_bin((c.y - lo.y) / L.y),
-                                      fraction_to_bin((c.z - lo.z) / L.z)) >> (30u - bits);
+        const uint32_t code = code_of(static_cast<uint32_t>(i));
         codes[i] = code;
         for (unsigned int p = 0; p < passes; ++p)
             radix::count_digit(s_hist + p * radix::kRadix, (code >> (p * radix::kBits)) & (radix::kRadix - 1));
@@ -1183,6 +1199,19 @@ __global__ void __launch_bounds__(256) query_codes(const float4* __restrict__ sp
     uint32_t* part = radix::hist_part(hist, passes);
     for (unsigned int j = threadIdx.x; j < passes * radix::kRadix; j += blockDim.x)
         if (s_hist[j]) atomicAdd(&part[j], s_hist[j]);
+    }
+
+//! The order of few queries in one launch (radix::kernel::rank_sort).
+__global__ void __launch_bounds__(radix::kernel::kRankBlock) query_order_ranked(const float4* __restrict__ spheres, const uint32_t n,
+                                                                                const float3* __restrict__ root_lo,
+                                                                                const float3* __restrict__ root_hi, const unsigned int bits,
+                                                                                uint32_t* __restrict__ order)
+    {
+    __shared__ radix::kernel::RankSort lds;
+    uint32_t code;
+    const uint32_t place = radix::kernel::rank_sort(lds, query_code(spheres, root_lo, root_hi, bits), n, blockIdx.x, code);
+    const uint32_t i = blockIdx.x * 64u + threadIdx.x;
+    if (threadIdx.x < 64u && i < n) order[place] = i;
     }
 
 //! Traversal by node fronts, one wave per 64 consecutive queries of the traversal order.  Blocks

@@ -113,6 +113,20 @@ __device__ __forceinline__ int common_prefix(const uint32_t* __restrict__ codes,
     return (ci == cj) ? 32 + __clz(static_cast<uint32_t>(i ^ j)) : __clz(ci ^ cj);
     }
 
+//! Morton code of primitive i (:28-52, :105-108).
+template<class InsertOpT>
+struct CodeOf
+    {
+    InsertOpT insert;
+    float3 lo, L;
+
+    __device__ __forceinline__ uint32_t of(const float3& c) const
+        {
+        return morton3(fraction_to_bin((c.x - lo.x) / L.x), fraction_to_bin((c.y - lo.y) / L.y), fraction_to_bin((c.z - lo.z) / L.z));
+        }
+    __device__ __forceinline__ uint32_t operator()(const uint32_t i) const { return of(insert.get(i).getCenter()); }
+    };
+
 //! Morton codes + radix digit histograms (+ clears of the per-build scratch words).
 template<class InsertOpT>
 __global__ void __launch_bounds__(256) lbvh_codes(const InsertOpT insert,
@@ -129,7 +143,7 @@ __global__ void __launch_bounds__(256) lbvh_codes(const InsertOpT insert,
     for (unsigned int j = threadIdx.x; j < passes * radix::kRadix; j += blockDim.x) s_hist[j] = 0u;
     __syncthreads();
 
-    const float3 L = make_float3(hi.x - lo.x, hi.y - lo.y, hi.z - lo.z);
+    const CodeOf<InsertOpT> code_of{insert, lo, make_float3(hi.x - lo.x, hi.y - lo.y, hi.z - lo.z)};
     const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
     const size_t first = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     // kUnroll independent primitive loads in flight per thread (few blocks keep the
@@ -149,9 +163,7 @@ __global__ void __launch_bounds__(256) lbvh_codes(const InsertOpT insert,
             {
             const size_t i = i0 + u * stride;
             if (i >= n) break;
-            const uint32_t code = morton3(fraction_to_bin((c[u].x - lo.x) / L.x),
-                                          fraction_to_bin((c[u].y - lo.y) / L.y),
-                                          fraction_to_bin((c[u].z - lo.z) / L.z));
+            const uint32_t code = code_of.of(c[u]);
             codes[i] = code;
             for (unsigned int p = 0; p < passes; ++p)
                 radix::count_digit(s_hist + p * radix::kRadix, (code >> (p * radix::kBits)) & (radix::kRadix - 1));
@@ -162,6 +174,27 @@ __global__ void __launch_bounds__(256) lbvh_codes(const InsertOpT insert,
     uint32_t* part = radix::hist_part(hist, passes);
     for (unsigned int j = threadIdx.x; j < passes * radix::kRadix; j += blockDim.x)
         if (s_hist[j]) atomicAdd(&part[j], s_hist[j]);
+    }
+
+//! lbvh_codes and the sort by counting (rank_sort): sorted codes and primitives (and the clears).
+template<class InsertOpT>
+__global__ void __launch_bounds__(radix::kernel::kRankBlock) lbvh_ranked_codes(const InsertOpT insert, const float3 lo, const float3 hi,
+                                                                               const uint32_t n, uint32_t* __restrict__ codes,
+                                                                               uint32_t* __restrict__ primitive,
+                                                                               uint32_t* __restrict__ clear, const size_t clear_words)
+    {
+    __shared__ radix::kernel::RankSort lds;
+    const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
+    for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < clear_words; i += stride) clear[i] = 0u;
+    uint32_t code;
+    const CodeOf<InsertOpT> code_of{insert, lo, make_float3(hi.x - lo.x, hi.y - lo.y, hi.z - lo.z)};
+    const uint32_t place = radix::kernel::rank_sort(lds, code_of, n, blockIdx.x, code);
+    const uint32_t i = blockIdx.x * 64u + threadIdx.x;
+    if (threadIdx.x < 64u && i < n)
+        {
+        codes[place] = code;
+        primitive[place] = i;
+        }
     }
 
 namespace bubble
@@ -505,13 +538,29 @@ struct SortedPointGather
  * of the nodes whose parents cross after the kernel boundary).  Only workgroup-scope
  * ordering is used; no global flag.
  */
-template<class InsertOpT, unsigned int CHUNK, unsigned int BLOCK>
-__global__ void __launch_bounds__(BLOCK) lbvh_bubble_chunk(const LBVHData tree,
-                                                                    const InsertOpT insert,
-                                                                    const int* __restrict__ range_end,
-                                                                    const uint32_t n,
-                                                                    const bool sorted_ready)
+template<class InsertOpT, unsigned int CHUNK>
+struct ChunkLds
     {
+    static constexpr bool kPointLeaves = detail::point_leaves<InsertOpT>::value;
+    float s_box[6][CHUNK];      //!< internal node cs + j
+    // point leaves keep no LDS copy: a thread holds its own leaves' points, and a sibling leaf's
+    // point is read back from the sorted points this workgroup wrote (72 KB of LDS for 2048
+    // leaves: two workgroups per CU); other leaves keep their boxes here
+    float s_leaf[kPointLeaves ? 1 : 6][kPointLeaves ? 1 : CHUNK];
+    uint32_t s_up[CHUNK];
+    int s_left[CHUNK];          //!< left child; sign bit: the node's range lies in the chunk
+    int s_right[CHUNK];
+    };
+
+template<class InsertOpT, unsigned int CHUNK, unsigned int BLOCK>
+__device__ __forceinline__ void bubble_chunk(ChunkLds<InsertOpT, CHUNK>& lds, const LBVHData& tree, const InsertOpT& insert,
+                                             const int* range_end, const uint32_t n, const bool sorted_ready, const uint32_t chunk)
+    {
+    auto& s_box = lds.s_box;
+    auto& s_leaf = lds.s_leaf;
+    auto& s_up = lds.s_up;
+    auto& s_left = lds.s_left;
+    auto& s_right = lds.s_right;
     constexpr int kInside = static_cast<int>(0x80000000u);
     constexpr bool kPointLeaves = detail::point_leaves<InsertOpT>::value;
     constexpr unsigned int kPer = CHUNK / BLOCK;                     // leaves per thread
@@ -522,18 +571,10 @@ __global__ void __launch_bounds__(BLOCK) lbvh_bubble_chunk(const LBVHData tree,
     constexpr uint32_t kArrival = 1u << 16;
     static_assert(CHUNK % BLOCK == 0, "whole leaves per thread");
     static_assert(CHUNK < kUpRoot, "chunk-relative parents in 16 bits");
-    __shared__ float s_box[6][CHUNK];   // internal node cs + j
-    // point leaves keep no LDS copy: a thread holds its own leaves' points, and a sibling leaf's
-    // point is read back from the sorted points this workgroup wrote (72 KB of LDS for 2048
-    // leaves: two workgroups per CU); other leaves keep their boxes here
-    __shared__ float s_leaf[kPointLeaves ? 1 : 6][kPointLeaves ? 1 : CHUNK];
-    __shared__ uint32_t s_up[CHUNK];
-    __shared__ int s_left[CHUNK];      // left child; sign bit: the node's range lies in the chunk
-    __shared__ int s_right[CHUNK];
     int lparent[kPer];                 // parents of this thread's leaves (same leaves in both loops)
     float3 lpoint[kPer];               // their points (point leaves)
 
-    const int cs = static_cast<int>(blockIdx.x * CHUNK);
+    const int cs = static_cast<int>(chunk * CHUNK);
     const int ce = min(cs + static_cast<int>(CHUNK), static_cast<int>(n));
     const int Ni = static_cast<int>(n) - 1;
     const int tid = static_cast<int>(threadIdx.x);
@@ -686,6 +727,58 @@ __global__ void __launch_bounds__(BLOCK) lbvh_bubble_chunk(const LBVHData tree,
         tree.lo[i] = make_float3(s_box[0][j], s_box[1][j], s_box[2][j]);
         tree.hi[i] = make_float3(s_box[3][j], s_box[4][j], s_box[5][j]);
         }
+    }
+
+template<class InsertOpT, unsigned int CHUNK, unsigned int BLOCK>
+__global__ void __launch_bounds__(BLOCK) lbvh_bubble_chunk(const LBVHData tree,
+                                                                    const InsertOpT insert,
+                                                                    const int* __restrict__ range_end,
+                                                                    const uint32_t n,
+                                                                    const bool sorted_ready)
+    {
+    __shared__ ChunkLds<InsertOpT, CHUNK> lds;
+    bubble_chunk<InsertOpT, CHUNK, BLOCK>(lds, tree, insert, range_end, n, sorted_ready, blockIdx.x);
+    }
+
+//! Leaves of the trees that one workgroup builds in one launch (one chunk).
+constexpr unsigned int kSmallTree = bubble::kChunk;
+
+//! The whole build of up to kSmallTree primitives by one workgroup: codes, sort, hierarchy (over
+//! the sorted codes in LDS) and boxes, each as the separate kernels make it.  A tree this small is
+//! all launches: 64 points took 51 us in eight, 20 in one, 1000 points 58 and 27, 2048 points 71
+//! and 41.
+template<class InsertOpT>
+__global__ void __launch_bounds__(radix::kernel::kSmallBlock) lbvh_small_build(const LBVHData tree, const InsertOpT insert, const float3 lo,
+                                                                               const float3 hi, const uint32_t n, uint32_t* __restrict__ codes,
+                                                                               const unsigned int passes, uint32_t* __restrict__ clear,
+                                                                               const size_t clear_words)
+    {
+    constexpr unsigned int ITEMS = kSmallTree / radix::kernel::kSmallBlock;
+    constexpr bool kGather = detail::point_leaves<InsertOpT>::value;
+    union Lds
+        {
+        __device__ Lds() {}
+        radix::kernel::SmallSort<ITEMS> sort;
+        ChunkLds<InsertOpT, kSmallTree> chunk;
+        };
+    __shared__ Lds lds;
+    for (size_t i = threadIdx.x; i < clear_words; i += blockDim.x) clear[i] = 0u;
+    radix::kernel::small_sort<ITEMS>(lds.sort, CodeOf<InsertOpT>{insert, lo, make_float3(hi.x - lo.x, hi.y - lo.y, hi.z - lo.z)}, n, passes);
+    const SpanLists none{};         // one chunk: no span passes
+    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x)
+        {
+        const uint32_t pid = lds.sort.vals[i];
+        codes[i] = lds.sort.keys[i];
+        tree.primitive[i] = pid;
+        if constexpr (kGather)
+            {
+            const float3 p = detail::insert_point(insert, pid, 0);
+            tree.sorted_points[i] = make_float4(p.x, p.y, p.z, __uint_as_float(pid));
+            }
+        hierarchy_node(tree, CodeKeys{lds.sort.keys, n}, static_cast<int>(i), none);
+        }
+    __syncthreads();                // the hierarchy's arrays, written by this workgroup; the sort's LDS is free
+    bubble_chunk<InsertOpT, kSmallTree, radix::kernel::kSmallBlock>(lds.chunk, tree, insert, tree.range_end, n, kGather, 0u);
     }
 
 namespace bubble

@@ -339,6 +339,174 @@ __global__ void __launch_bounds__(kBlock) onesweep_pass(const KeyT* __restrict__
         }
     }
 
+constexpr unsigned int kSmallBlock = 1024;
+constexpr unsigned int kSmallWaves = kSmallBlock / 64;
+//! LDS of a one-workgroup sort of at most kSmallBlock * ITEMS keys.
+template<unsigned int ITEMS>
+struct SmallSort
+    {
+    uint32_t keys[kSmallBlock * ITEMS];
+    uint32_t vals[kSmallBlock * ITEMS];
+    uint32_t wave[kSmallWaves][kRadix];     //!< digit counts of each wave, then their first places
+    uint32_t tmp[kRadix / 64];
+    };
+
+//! Stable sort of n keys (key(i), identity values) by one workgroup of kSmallBlock threads, all
+//! passes in LDS: the result is in lds.keys / lds.vals (synchronized).
+/*!
+ * Ranking as in onesweep_pass (ballots within a wave, wave counters), the waves' places from one
+ * scan over the digits.
+ */
+template<unsigned int ITEMS, class KeyFn>
+__device__ __forceinline__ void small_sort(SmallSort<ITEMS>& lds, const KeyFn& key, const uint32_t n, const unsigned int passes)
+    {
+    const unsigned int tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t first = wave * 64u * ITEMS + lane;
+    uint32_t k[ITEMS], v[ITEMS], r[ITEMS];
+    #pragma unroll
+    for (unsigned int i = 0; i < ITEMS; ++i)
+        {
+        v[i] = first + 64u * i;
+        k[i] = v[i] < n ? key(v[i]) : ~0u;      // keys past the end carry the last digits and stay last
+        }
+    const uint64_t below = (lane == 0u) ? 0ull : (~0ull >> (64u - lane));
+    for (unsigned int p = 0; p < passes; ++p)
+        {
+        const unsigned int shift = p * kBits;
+        for (unsigned int j = tid; j < kSmallWaves * kRadix; j += kSmallBlock) (&lds.wave[0][0])[j] = 0u;
+        __syncthreads();
+        #pragma unroll
+        for (unsigned int i = 0; i < ITEMS; ++i)
+            {
+            const uint32_t d = (k[i] >> shift) & (kRadix - 1u);
+            uint64_t same = ~0ull;
+            #pragma unroll
+            for (unsigned int b = 0; b < kBits; ++b)
+                {
+                const bool bit = (d >> b) & 1u;
+                const uint64_t bal = __builtin_amdgcn_ballot_w64(bit);
+                same &= bit ? bal : ~bal;
+                }
+            const uint32_t before = static_cast<uint32_t>(__popcll(same & below));
+            const uint32_t prev = lds.wave[wave][d];
+            r[i] = prev + before;
+            if (before == 0u) lds.wave[wave][d] = prev + static_cast<uint32_t>(__popcll(same));
+            }
+        __syncthreads();
+        // thread d: places of digit d's keys, wave by wave
+        uint32_t total = 0u, incl = 0u;
+        if (tid < kRadix)
+            {
+            #pragma unroll
+            for (unsigned int w = 0; w < kSmallWaves; ++w)
+                {
+                const uint32_t c = lds.wave[w][tid];
+                lds.wave[w][tid] = total;
+                total += c;
+                }
+            incl = total;
+            #pragma unroll
+            for (unsigned int d = 1; d < 64; d <<= 1)
+                {
+                const uint32_t y = __shfl_up(incl, d, 64);
+                if (lane >= d) incl += y;
+                }
+            if (lane == 63u) lds.tmp[wave] = incl;
+            }
+        __syncthreads();
+        if (tid < kRadix)
+            {
+            uint32_t base = incl - total;
+            for (unsigned int w = 0; w < wave; ++w) base += lds.tmp[w];
+            #pragma unroll
+            for (unsigned int w = 0; w < kSmallWaves; ++w) lds.wave[w][tid] += base;
+            }
+        __syncthreads();
+        #pragma unroll
+        for (unsigned int i = 0; i < ITEMS; ++i)
+            {
+            const uint32_t pos = lds.wave[wave][(k[i] >> shift) & (kRadix - 1u)] + r[i];
+            lds.keys[pos] = k[i];
+            lds.vals[pos] = v[i];
+            }
+        __syncthreads();
+        if (p + 1u < passes)
+            {
+            #pragma unroll
+            for (unsigned int i = 0; i < ITEMS; ++i)
+                {
+                k[i] = lds.keys[first + 64u * i];
+                v[i] = lds.vals[first + 64u * i];
+                }
+            }
+        }
+    }
+
+//! Sort by counting: place of each of a workgroup's 64 keys = the number of keys that come before
+//! it (smaller, or equal and of a lower index), every pair of keys compared.
+/*!
+ * For few keys n^2 comparisons by the whole chip in one launch cost less than a launch per digit:
+ * two instructions per comparison (compare and add with carry, the other key broadcast from LDS,
+ * four per read), the keys made anew by every workgroup.  Wave w compares with the 64-key chunks
+ * w, w + kRankWaves, ...; the waves' counts are added in LDS.  A build with it against one with
+ * codes and four digit passes (five launches): 4096 points 51 us against 81, 10,000 63 against
+ * 87, 16,384 73 against 90; at 20,000 the comparisons have caught up (91 with the passes).  All
+ * passes in one workgroup's LDS took 44 us for 10,000 keys, as long as the five launches.
+ *
+ * Keys of up to 30 bits: 2 key + 1 and 2 key as thresholds tell ties of lower from ties of higher
+ * index.  Returns the calling lane's place (wave 0 only; lanes with i < n) and its key in `mine`.
+ */
+constexpr unsigned int kRankWaves = 16;
+constexpr unsigned int kRankBlock = 64 * kRankWaves;
+//! Keys up to which counting is the faster sort (figures above).
+constexpr unsigned int kRankSort = 16384;
+
+struct RankSort
+    {
+    alignas(16) uint32_t keys[kRankWaves][64];
+    uint32_t count[kRankWaves][64];
+    };
+
+template<class KeyFn>
+__device__ __forceinline__ uint32_t rank_sort(RankSort& lds, const KeyFn& key, const uint32_t n, const uint32_t tile, uint32_t& mine)
+    {
+    const unsigned int lane = threadIdx.x & 63u;
+    const unsigned int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t i = tile * 64u + lane;
+    mine = i < n ? key(i) : 0u;
+    const uint32_t chunks = (n + 63u) / 64u;
+    uint32_t count = 0u;
+    uint32_t next = wave * 64u + lane < n ? key(wave * 64u + lane) : 0x7FFFFFFFu;
+    for (uint32_t c = wave; c < chunks; c += kRankWaves)
+        {
+        uint32_t* buf = lds.keys[wave];
+        buf[lane] = 2u * next;                                  // past the end: above every threshold
+        const uint32_t j = (c + kRankWaves) * 64u + lane;
+        next = j < n ? key(j) : 0x7FFFFFFFu;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wave's own words, in order
+        if (c != tile)
+            {
+            const uint32_t t = 2u * mine + (c < tile ? 1u : 0u);
+            #pragma unroll
+            for (unsigned int l = 0; l < 64; ++l) count += buf[l] < t ? 1u : 0u;
+            }
+        else
+            {
+            #pragma unroll 1
+            for (unsigned int l = 0; l < 64; ++l)
+                count += buf[l] < 2u * mine + (l < lane ? 1u : 0u) ? 1u : 0u;
+            }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+    lds.count[wave][lane] = count;
+    __syncthreads();
+    if (wave) return 0u;
+    uint32_t place = 0u;
+    #pragma unroll
+    for (unsigned int w = 0; w < kRankWaves; ++w) place += lds.count[w][lane];
+    return place;
+    }
+
 } // end namespace kernel
 
 //! Run all passes.  Keys/values start in (keys, vals); the sorted result ends in
