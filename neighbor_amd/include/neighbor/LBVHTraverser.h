@@ -12,9 +12,8 @@
 // ExactSphereQueryOp (with the float SphereQueryOp it reports fewer, tighter hits than the
 // reference); Wave (ExactSphereQueryOp only) exact-box records with bucket leaves; WaveQuantized
 // the same over decoded quantized boxes, for SphereQueryOp (results identical to Quantized) and
-// ExactSphereQueryOp.  SphereQueryOp in every variant and ExactSphereQueryOp in the wave variants
-// walk by node fronts (kernels/FrontWalk.h); other query ops, and ExactSphereQueryOp in the rope
-// variants, take one rope path per query.
+// ExactSphereQueryOp.  Both queries walk by node fronts (kernels/FrontWalk.h) in every variant;
+// other query ops (rope variants) take one rope path per query.
 #ifndef NEIGHBOR_LBVH_TRAVERSER_H_
 #define NEIGHBOR_LBVH_TRAVERSER_H_
 
@@ -459,7 +458,8 @@ template<class QueryOpT, class OutputOpT, class TranslateOpT, class TransformOpT
 void LBVHTraverser::traverse(const LaunchParameters& params, const LBVH& lbvh, const QueryOpT& query,
                              const OutputOpT& out, const TranslateOpT& images, const TransformOpT& transform)
     {
-    if constexpr (gpu::kernel::wave::places_rows<OutputOpT>::value)
+    constexpr bool placed = gpu::kernel::wave::places_rows<OutputOpT>::value;
+    if constexpr (placed)
         if (m_variant != TraversalVariant::Wave && m_variant != TraversalVariant::WaveQuantized)
             throw std::invalid_argument("PlacedRowPairOp: rows are placed by the wave traversal variants only");
     if (lbvh.getN() == 0) return;
@@ -470,32 +470,27 @@ void LBVHTraverser::traverse(const LaunchParameters& params, const LBVH& lbvh, c
 
     const unsigned int* order = (m_order && m_order_n == query.size()) ? m_order : nullptr;
     const dim3 grid(div_up(query.size(), block));
-    constexpr bool reference = std::is_same<QueryOpT, SphereQueryOp>::value;
-    if constexpr (reference)
+    if (m_variant == TraversalVariant::Wave || m_variant == TraversalVariant::WaveQuantized)
+        {
+        traverse_wave(params, lbvh, query, out, images, transform, order);
+        }
+    else if constexpr (placed)
+        {
+        // refused above
+        }
+    else if constexpr (std::is_same<QueryOpT, SphereQueryOp>::value || std::is_same<QueryOpT, ExactSphereQueryOp>::value)
         {
         if (m_variant == TraversalVariant::Quantized)
-            {
             launch_front(params, query, out, images, order, lbvh.getNNodes(),
                          gpu::kernel::front::QuantizedSource{m_data.get(), float3(), float3(), float3(), lbvh.getNInternal()});
-            check_launch("lbvh_traverse");
-            return;
-            }
-        if (m_variant == TraversalVariant::FloatRope || m_variant == TraversalVariant::FloatRopeExact)
-            {
+        else
             launch_front(params, query, out, images, order, lbvh.getNNodes(),
                          gpu::kernel::front::RopeSource{m_float.get(), lbvh.getNInternal()});
-            check_launch("lbvh_traverse");
-            return;
-            }
         }
-    if (m_variant == TraversalVariant::Quantized)
+    else if (m_variant == TraversalVariant::Quantized)
         {
         hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_ropes<OutputOpT, QueryOpT, TranslateOpT>), grid, dim3(block), 0,
                            params.stream, out, data(), query, images, order, lbvh.getNNodes());
-        }
-    else if (m_variant == TraversalVariant::Wave || m_variant == TraversalVariant::WaveQuantized)
-        {
-        traverse_wave(params, lbvh, query, out, images, transform, order);
         }
     else
         {

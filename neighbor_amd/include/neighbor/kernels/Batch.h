@@ -306,7 +306,7 @@ __device__ __forceinline__ void batch_traverse_body(const OutputOpT& out,
                 const Source src{nodes, points, primitive, NullTransformOp(), n_internal};
                 front::FrontWave& W = *reinterpret_cast<front::FrontWave*>(lds[wid]);
                 front::FrontPairs& P = *reinterpret_cast<front::FrontPairs*>(lds[wid] + sizeof(front::FrontWave));
-                const bool walked = !rooted || (front::takes<QueryOpT>(valid, qd, images, root_box)
+                const bool walked = !rooted || (front::takes<Source, QueryOpT>(valid, qd, images, root_box)
                     && front::walk<false>(out, src, root, root_box, query, images, valid, idx, qd, 2u * nb - 1u, W, P, nullptr));
                 if (valid && !rooted) out.finalize(out.setup(idx, qd));
                 else if (valid && !walked) front::lane_walk(out, src, root, stop, root_box, query, images, idx, qd, n_nodes);

@@ -125,11 +125,28 @@ struct BucketSource
     __device__ __forceinline__ uint32_t value(const unsigned int l, const Node&) const { return transform(primitive[l]); }
     //! Point of a leaf and its value for the output op (exact query).
     __device__ __forceinline__ float4 point(const ExactSphereQueryOp&, const unsigned int l) const { return points[l]; }
+    __device__ __forceinline__ float4 point(const ExactSphereQueryOp&, const unsigned int l, const BoundingBox&, bool& inside) const
+        {
+        inside = true;
+        return points[l];
+        }
     __device__ __forceinline__ uint32_t point_value(const float4& p) const { return transform(__float_as_uint(p.w)); }
     __device__ __forceinline__ float error() const { return 0.0f; }
     };
 
-//! Float rope records of decoded quantized boxes: a negative word is a leaf's value.
+//! The point that an exact query holds for a leaf's value (w: the value), and whether it lies in
+//! the leaf's box and the root's.
+__device__ __forceinline__ float4 value_point(const ExactSphereQueryOp& query, const uint32_t value)
+    {
+    const float* p = query.points + static_cast<size_t>(query.stride) * value;
+    return make_float4(p[0], p[1], p[2], __uint_as_float(value));
+    }
+__device__ __forceinline__ bool holds(const BoundingBox& b, const float4& p)
+    {
+    return p.x >= b.lo.x && p.x <= b.hi.x && p.y >= b.lo.y && p.y <= b.hi.y && p.z >= b.lo.z && p.z <= b.hi.z;
+    }
+
+//! Float rope records: a negative word is a leaf's value.
 struct RopeSource
     {
     static constexpr bool kFirst = true;
@@ -148,6 +165,17 @@ struct RopeSource
         return BoundingBox(r.lo, r.hi);
         }
     __device__ __forceinline__ uint32_t value(const unsigned int, const Node& r) const { return ~static_cast<uint32_t>(r.lf); }
+    __device__ __forceinline__ float4 point(const ExactSphereQueryOp& query, const unsigned int l) const
+        {
+        return value_point(query, ~__float_as_uint(nodes[2u * (n_internal + l)].w));
+        }
+    __device__ __forceinline__ float4 point(const ExactSphereQueryOp& query, const unsigned int l, const BoundingBox& root_box, bool& inside) const
+        {
+        const float4 p = point(query, l);
+        inside = holds(box(n_internal + l), p) && holds(root_box, p);
+        return p;
+        }
+    __device__ __forceinline__ uint32_t point_value(const float4& p) const { return __float_as_uint(p.w); }
     __device__ __forceinline__ float error() const { return 0.0f; }
     };
 
@@ -179,6 +207,17 @@ struct QuantizedSource
         return detail::decode_box(static_cast<uint32_t>(r.x), static_cast<uint32_t>(r.y), rlo, rhi, bins);
         }
     __device__ __forceinline__ uint32_t value(const unsigned int, const Node& r) const { return ~static_cast<uint32_t>(r.lf); }
+    __device__ __forceinline__ float4 point(const ExactSphereQueryOp& query, const unsigned int l) const
+        {
+        return value_point(query, ~static_cast<uint32_t>(data[n_internal + l].z));
+        }
+    __device__ __forceinline__ float4 point(const ExactSphereQueryOp& query, const unsigned int l, const BoundingBox& root_box, bool& inside) const
+        {
+        const float4 p = point(query, l);
+        inside = holds(box(n_internal + l), p) && holds(root_box, p);
+        return p;
+        }
+    __device__ __forceinline__ uint32_t point_value(const float4& p) const { return __float_as_uint(p.w); }
     //! The defined decoding rounds the product (at most 1023 bins, within an ulp of the box's
     //! side) and the sum down or up by an ulp each, the plain one the sum to nearest: together
     //! below 4 2^-23 of (largest corner + side).
@@ -530,7 +569,8 @@ __device__ __forceinline__ void write_hits(unsigned int* __restrict__ neigh, uns
  * in float, against the radius padded by R 2^-20 + 2^-20 (largest coordinate + largest image
  * component) + twice the boxes' own error: each of the three roundings per axis errs by at most
  * 2^-24 of a magnitude below that sum (and the reference query's directed roundings admit at
- * most 15 2^-24 more of R^2), so a box with a hit always passes.
+ * most 15 2^-24 more of R^2; 2^-120 covers squares below the range of float), so a box with a
+ * hit always passes.
  *
  * Leaf tests, exact query: with o the wave's origin of the image (float), q' = fl((q + t) - o)
  * and p' = fl(p - o), the value s = |p'|^2 - 2 p'.q' + (|q'|^2 - R^2) computed in float differs
@@ -538,6 +578,12 @@ __device__ __forceinline__ void write_hits(unsigned int* __restrict__ neigh, uns
  * roundings of |p'|^2, five sums of terms that stay below 4 B^2, taken as truncated, and the
  * roundings of p' and q' times 2 R); farther leaves have s > 0 by more than their own error.
  * |s| > band = 2^-18 B^2 is therefore decided by the sign; the others by the FP64 definition.
+ *
+ * Rope and quantized records hold a leaf's value only, and the exact query its own point of it.
+ * A point in the leaf's box and the root's is decided as above (its boxes' conservative tests
+ * pass where the point is a hit); any other point by the query's box and point tests, which
+ * admit boxes up to R 2^-20 + 2^-21 (largest coordinate) and roundings farther than R: such
+ * walks pad by 2^-18 in place of 2^-20.
  *
  * Reference query: p is the center of the leaf's box, h a bound of the batch's half diagonals.
  * The box is a hit if the center is (distance <= R) and a miss if the center is farther than
@@ -557,6 +603,8 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
     constexpr bool kExact = std::is_same<QueryOpT, ExactSphereQueryOp>::value;
     constexpr bool kCount = std::is_same<OutputOpT, CountNeighborsOp>::value;
     constexpr bool kRows = Rows<OutputOpT>::kOn;
+    constexpr bool kChecked = kExact && SrcT::kFirst;   // points come from the query: any may lie outside of its leaf's box
+    constexpr float kPad = kChecked ? 0x1p-18f : 0x1p-20f;
     static_assert(!TEAM || kCount || kRows, "teams count or write rows");
     const unsigned int lane = threadIdx.x & 63u;
     const unsigned int member = TEAM ? static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6))) : 0u;
@@ -595,10 +643,10 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
         const float3 uhi = make_float3(-over_rows_min(-ghi.x), -over_rows_min(-ghi.y), -over_rows_min(-ghi.z));
         const float cmax = fmaxf(fmaxf(fmaxf(fabsf(ulo.x), fabsf(uhi.x)), fmaxf(fabsf(ulo.y), fabsf(uhi.y))),
                                  fmaxf(fabsf(ulo.z), fabsf(uhi.z)));
-        const float pad = 0x1p-20f * (cmax + tmax) + 2.0f * src.error();
+        const float pad = kPad * (cmax + tmax) + 2.0f * src.error();
         const auto padded = [&](const float radius) {
-            const float R = radius * (1.0f + 0x1p-20f) + pad;
-            return R * R * (1.0f + 0x1p-19f);
+            const float R = radius * (1.0f + kPad) + pad;
+            return R * R * (1.0f + 0x1p-19f) + 0x1p-120f;
         };
         W.sphere[lane] = make_float4(q.x, q.y, q.z, act ? padded(r) : -1.0f);
         if ((lane & 3u) == 0u)
@@ -654,6 +702,7 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
         float half = 0.0f;                      // their bound of the leaf boxes' half diagonals
         float3 o = make_float3(0.0f, 0.0f, 0.0f);
         uint32_t cnt[4] = {0u, 0u, 0u, 0u};
+        uint32_t odd_hits = 0u;                 // kChecked, counts: hits outside of their leaves' boxes
         unsigned long long run0 = 0ull;
         unsigned int round = 0u;
         // each step settles at least its first entry, and every image visits a node at most once
@@ -846,11 +895,12 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
                     float px = 0.0f, py = 0.0f, pz = 0.0f;
                     uint32_t value = 0u;
                     float reach2 = 0.0f;
+                    bool inside = true;
                     if (has)
                         {
                         if constexpr (kExact)
                             {
-                            const float4 p = src.point(query, leaf);
+                            const float4 p = src.point(query, leaf, root_box, inside);
                             px = p.x;
                             py = p.y;
                             pz = p.z;
@@ -893,7 +943,7 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
                         }
                     float x = px - o.x, y = py - o.y, z = pz - o.z;
                     float w = fmaf(z, z, fmaf(y, y, x * x));
-                    if (!has || !(w < kFarLeaf))
+                    if (!has || !inside || !(w < kFarLeaf))
                         {
                         x = y = z = 0.0f;
                         w = kNever;
@@ -922,6 +972,20 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
                             {
                             #pragma unroll
                             for (unsigned int g = 0; g < 4; ++g) cnt[g] += static_cast<uint32_t>(__popc(acc[g]));
+                            }
+                        if constexpr (kChecked)
+                            {
+                            // the others by the query's own tests
+                            for (unsigned long long odd = wave::vote(has && !inside); odd; odd &= odd - 1ull)
+                                {
+                                const unsigned int b = static_cast<unsigned int>(__builtin_ctzll(odd));
+                                const unsigned int l = static_cast<unsigned int>(__builtin_amdgcn_readlane(static_cast<int>(leaf), static_cast<int>(b)));
+                                const ExactSphere v = query.get(anew(q), images.get(k));
+                                const bool in = act && query.overlap(v, root_box) && query.overlap(v, src.box(n_internal + l))
+                                                && ExactSphereQueryOp::refine_point(v, src.point(query, l));
+                                if constexpr (kCount) odd_hits += in ? 1u : 0u;
+                                else hits |= in ? 1ull << b : 0ull;
+                                }
                             }
                         }
                     else
@@ -1025,6 +1089,7 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
                     c += static_cast<uint32_t>(__shfl_xor(static_cast<int>(c), 32, 64));
                     if ((lane >> 4) == g) mine = c;
                     }
+                if constexpr (kChecked) mine += odd_hits;
                 }
             if constexpr (TEAM)
                 {
@@ -1069,9 +1134,9 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
     return true;
     }
 
-//! True when every lane's query and every image vector (reference query: and the root box, which
-//! holds every box) take the walk above (wave-uniform).
-template<class QueryOpT, class TranslateOpT>
+//! True when every lane's query and every image vector (reference query, quantized boxes: and the
+//! root box, which holds every box) take the walk above (wave-uniform).
+template<class SrcT, class QueryOpT, class TranslateOpT>
 __device__ __forceinline__ bool takes(const bool valid, const float4& q, const TranslateOpT& images, const BoundingBox& root_box)
     {
     const unsigned int lane = threadIdx.x & 63u;
@@ -1085,7 +1150,7 @@ __device__ __forceinline__ bool takes(const bool valid, const float4& q, const T
         const double3 t = as_double3(images.get(lane));
         ok = ok && small(static_cast<float>(t.x), static_cast<float>(t.y), static_cast<float>(t.z));
         }
-    if constexpr (!std::is_same<QueryOpT, ExactSphereQueryOp>::value)
+    if constexpr (SrcT::kFirst || !std::is_same<QueryOpT, ExactSphereQueryOp>::value)
         ok = ok && small(root_box.lo.x, root_box.lo.y, root_box.lo.z) && small(root_box.hi.x, root_box.hi.y, root_box.hi.z);
     return wave::vote(!ok) == 0ull;
     }
@@ -1247,7 +1312,7 @@ lbvh_traverse_front(const OutputOpT out,
     front::bind(src, root_box, bins);
     front::FrontWave& W = *reinterpret_cast<front::FrontWave*>(lds[wid]);
     front::FrontPairs& P = *reinterpret_cast<front::FrontPairs*>(lds[wid] + sizeof(front::FrontWave));
-    if (front::takes<QueryOpT>(valid, q, images, root_box)
+    if (front::takes<SrcT, QueryOpT>(valid, q, images, root_box)
         && front::walk<false>(out, src, root, root_box, query, images, valid, idx, q, n_nodes, W, P, nullptr)) return;
     if (valid)
         front::lane_walk(out, src, root, LBVHSentinel, root_box, query, images, idx, q, n_nodes);
@@ -1284,7 +1349,7 @@ lbvh_traverse_team(const OutputOpT out,
     front::bind(src, root_box, bins);
     front::FrontWave& W = *reinterpret_cast<front::FrontWave*>(lds[wid]);
     front::FrontPairs& P = *reinterpret_cast<front::FrontPairs*>(lds[wid] + sizeof(front::FrontWave));
-    if (front::takes<QueryOpT>(valid, q, images, root_box)
+    if (front::takes<SrcT, QueryOpT>(valid, q, images, root_box)
         && front::walk<true>(out, src, root, root_box, query, images, valid, idx, q, n_nodes, W, P, &team)) return;
     if (valid && wid == 0u)
         front::lane_walk(out, src, root, LBVHSentinel, root_box, query, images, idx, q, n_nodes);

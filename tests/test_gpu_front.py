@@ -221,3 +221,75 @@ def test_batch_grids(nb, orc, grid):
         a = np.lexsort((nj[rows], nk[rows], i))
         c = np.lexsort((ref["j"], ref["k"], i))
         assert np.array_equal(nk[rows][a], ref["k"].astype(np.int64)[c]) and np.array_equal(nj[rows][a] - s, ref["j"].astype(np.int64)[c])
+
+
+@pytest.mark.parametrize("n", [1, 2, 31, 33, 64, 65, 500, 2049])
+def test_exact_query_rope_records(nb, orc, n):
+    """Exact rows of the rope variants, whose records hold the leaves' values only: the pairs of the
+    FP64 sum over all points, in the rope walk's order, with and without a transform map."""
+    import torch
+    from neighbor_amd.api import exact_rows, exclusive_scan
+    from neighbor_amd.workloads import images27
+    rng = np.random.default_rng(n + 5)
+    pts, L = points_of(n, rng, "lattice" if n % 2 else "uniform")
+    r = 1.5
+    sph = np.concatenate([pts, np.full((n, 1), r, np.float32)], 1).astype(np.float32)
+    sph[::5, 3] = 0.0
+    sph[1::9, 3] = np.float32(0.45 * L)
+    ref = orc.exact_bruteforce(pts, sph, images27(L, dtype=np.float64))
+    counts = ref["counts"].astype(np.int64)
+    d_sph = torch.from_numpy(sph).cuda()
+    d_img = torch.from_numpy(images27(L, dtype=np.float64)).cuda()
+    lb = nb.LBVH()
+    lb.build(torch.from_numpy(pts).cuda(), [0, 0, 0], [L] * 3)
+    prim = host(lb.arrays()["primitive"]).view(np.uint32).astype(np.int64)
+    place = np.empty(n, np.int64)
+    place[prim] = np.arange(n)
+    tag = rng.permutation(n + 3)[:n].astype(np.int32)       # values of the points, and the points by value
+    by_tag = np.full((n + 3, 3), 1e6, np.float32)
+    by_tag[tag] = pts
+    for variant in (nb.NB_VARIANT_QUANTIZED, nb.NB_VARIANT_FLOAT_ROPE, nb.NB_VARIANT_FLOAT_ROPE_EXACT):
+        for mapped in (False, True):
+            tr = nb.LBVHTraverser(variant=variant)
+            kw = dict(transform_map=torch.from_numpy(tag).cuda()) if mapped else {}
+            d_pts = torch.from_numpy(by_tag if mapped else pts).cuda()
+            for order in (None, lb.device_pointers()["primitive"]):
+                got = tr.exact_count(lb, d_sph, d_pts, images=d_img, order=order, **kw)
+                assert np.array_equal(host(got).view(np.uint32), ref["counts"])
+                start = exclusive_scan(got)
+                total = int(counts.sum())
+                neigh = torch.full((total + 1,), -1, dtype=torch.int32, device="cuda")
+                img = torch.full((total + 1,), 77, dtype=torch.uint8, device="cuda")
+                exact_rows(tr, lb, d_sph, d_pts, start, got, neigh, img, images=d_img, order=order, **kw)
+                i = np.repeat(np.arange(n), counts)
+                key = np.lexsort((place[ref["j"]], ref["k"], ref["i"] if "i" in ref else i))
+                want_j = ref["j"].astype(np.int64)[key]
+                assert np.array_equal(host(img)[:-1].astype(np.int64), ref["k"].astype(np.int64)[key])
+                assert np.array_equal(host(neigh)[:-1].astype(np.int64), tag[want_j] if mapped else want_j)
+
+
+@pytest.mark.parametrize("n", [1, 3, 40, 700])
+def test_exact_query_other_points(nb, n):
+    """Points that need not lie in the tree's boxes: a hit is a point within the radius whose leaf's
+    box is, too (the quantized boxes: up to two bins larger)."""
+    import torch
+    rng = np.random.default_rng(n + 11)
+    L = 9.0
+    centers = (rng.random((n, 3)) * L).astype(np.float32)
+    other = (centers + rng.normal(0, 0.6, (n, 3))).astype(np.float32)
+    other[::9, 1] = np.nan
+    other[4::9] = centers[4::9]
+    nq = 200
+    sph = np.concatenate([rng.random((nq, 3)) * L, rng.uniform(0.2, 2.5, (nq, 1))], 1).astype(np.float32)
+    box_r = 0.25
+    lb = nb.LBVH()
+    lb.build(torch.from_numpy(centers).cuda(), [0, 0, 0], [L] * 3, radius=box_r)
+    q, R = sph[:, None, :3].astype(np.float64), sph[:, None, 3].astype(np.float64)
+    near = ((q - other[None].astype(np.float64)) ** 2).sum(2) <= R * R
+    gap = np.sqrt((np.maximum(np.abs(q - centers[None]) - box_r, 0.0) ** 2).sum(2))
+    least = (near & (gap <= R - 1e-4)).sum(1)
+    for variant, more in ((nb.NB_VARIANT_FLOAT_ROPE_EXACT, 1e-4), (nb.NB_VARIANT_FLOAT_ROPE, 0.06), (nb.NB_VARIANT_QUANTIZED, 0.06)):
+        tr = nb.LBVHTraverser(variant=variant)
+        got = host(tr.exact_count(lb, torch.from_numpy(sph).cuda(), torch.from_numpy(other).cuda())).astype(np.int64)
+        most = (near & (gap <= R + more)).sum(1)
+        assert (got >= least).all() and (got <= most).all()
