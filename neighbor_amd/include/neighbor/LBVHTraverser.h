@@ -314,7 +314,7 @@ class LBVHTraverser : public Tunable<unsigned int>
             if constexpr (teams)
                 if (n <= kTeamQueries)
                     {
-                    const unsigned int per = n <= kTeamQueries / 4u ? 16u : n <= kTeamQueries / 2u ? 32u : 64u;
+                    const unsigned int per = n <= kTeamQueries / 16u ? 4u : n <= kTeamQueries / 4u ? 16u : n <= kTeamQueries / 2u ? 32u : 64u;
                     hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_team<SourceT, OutputOpT, QueryOpT, TranslateOpT>),
                                        dim3(div_up(n, per)), dim3(256), 0, params.stream, out, src, m_lbvh_lo.get(), m_lbvh_hi.get(),
                                        m_bins.get(), m_root, query, images, order, n_nodes, per);
@@ -378,10 +378,12 @@ class LBVHTraverser : public Tunable<unsigned int>
         //! images: 256 queries 44 us and 44, 512 71 and 54, 1000 89 and 44; without images 14 and 24,
         //! 21 and 30, 34 and 33; 10^6 (one rope path per lane) 8.2 ms and 0.7.
         static constexpr unsigned int kSortQueries = 256;
-        //! Queries up to which four waves serve 64, 32 or 16 queries together: one wave's chain of
+        //! Queries up to which four waves serve 64, 32, 16 or 4 queries together: one wave's chain of
         //! steps takes longer than the chip needs for all of them.  Exact count and fill of 10,000
         //! points (27 images): 82 and 115 us with a wave per 64 queries, 48 and 61 with teams for
-        //! 16; of 131,071 points (no images) 90 and 125 us with waves, 201 and 229 with teams.
+        //! 16; of 131,071 points (no images) 90 and 125 us with waves, 201 and 229 with teams.  Teams
+        //! for 16 and for 4: 1000 points 35 and 47 us, 29 and 38; 4000 points 56 and 72, 45 and 56;
+        //! 8000 points 48 and 65, 62 and 77.
         static constexpr unsigned int kTeamQueries = 1u << 16;
         //! Tail split (wave::tail_block): per XCD, the last m_tail_groups groups of 256 queries run
         //! as m_tail_split blocks each, so that the waves that start last are shorter.  Exact count
