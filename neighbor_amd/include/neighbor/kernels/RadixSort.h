@@ -6,8 +6,10 @@
 // (key, original index).
 //
 // Design (one kernel per 8-bit digit pass, "onesweep" style):
-//  * A tile is 512 threads x 12 keys = 6144 keys, held in registers in a
-//    wave-striped arrangement (key w*768 + i*64 + lane of the tile lives in lane
+//  * A tile is 512 threads x 12 keys = 6144 keys (512 x 4 up to kShortKeys keys, where
+//    6144-key tiles leave most CUs without one: four passes at 50,000 keys take 13 us less with 4
+//    than with 12, at 131,071 10, at 300,000 4; at 10^6 15 us more), held in registers in a
+//    wave-striped arrangement (key w*64*items + i*64 + lane of the tile lives in lane
 //    `lane` of wave w, item i), so loads are coalesced and (wave, item, lane)
 //    order is input order.
 //  * Ranking inside a wave64 uses eight ballots per key to find the lanes holding
@@ -46,12 +48,14 @@ constexpr unsigned int kBits = 8;
 constexpr unsigned int kRadix = 1u << kBits;
 constexpr unsigned int kBlock = 512;                 // threads per tile (the first kRadix own a digit each)
 constexpr unsigned int kWaves = kBlock / 64;
-constexpr unsigned int kItems = 12;                  // keys per thread (512 x 8: -3% at 64M; 256 x 16: 140 VGPRs)
-constexpr unsigned int kTile = kBlock * kItems;      // 6144 keys
+// keys per thread, by the number of keys
+constexpr unsigned int kItems = 12, kShortItems = 4;
+constexpr size_t kShortKeys = 3u << 17;
 constexpr uint32_t kFlagAggregate = 1u << 30;
 constexpr uint32_t kFlagPrefix = 2u << 30;
 constexpr uint32_t kValueMask = (1u << 30) - 1u;
 constexpr uint32_t kSpinLimit = 1u << 22;
+constexpr unsigned int kWindow = 8;                  // earlier tiles whose counts are read at once
 
 static_assert(kBlock % kRadix == 0 && kBlock >= kRadix, "one thread per digit in the look-back");
 
@@ -61,7 +65,11 @@ static_assert(kBlock % kRadix == 0 && kBlock >= kRadix, "one thread per digit in
 constexpr unsigned int kHistParts = 8;
 
 inline unsigned int num_passes(unsigned int end_bit) { return (end_bit + kBits - 1) / kBits; }
-inline unsigned int num_tiles(size_t n) { return static_cast<unsigned int>((n + kTile - 1) / kTile); }
+inline unsigned int num_tiles(size_t n)
+    {
+    const size_t tile = kBlock * (n <= kShortKeys ? kShortItems : kItems);
+    return static_cast<unsigned int>((n + tile - 1) / tile);
+    }
 
 //! Words of device workspace for a sort of n keys over end_bit bits.
 /*!
@@ -83,7 +91,9 @@ struct Workspace
     static size_t words(size_t n, unsigned int end_bit)
         {
         const unsigned int p = num_passes(end_bit);
-        return header_words(p) + static_cast<size_t>(p) * num_tiles(n) * kRadix;
+        // no fewer than any smaller n takes
+        const unsigned int tiles = num_tiles(n), small = num_tiles(n <= kShortKeys ? n : kShortKeys);
+        return header_words(p) + static_cast<size_t>(p) * (tiles > small ? tiles : small) * kRadix;
         }
     static Workspace carve(uint32_t* base, size_t n, unsigned int end_bit)
         {
@@ -180,7 +190,7 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s
     }
 
 //! One stable 8-bit digit pass.  IDENTITY_VALUES: values are the input positions (not read).
-template<bool IDENTITY_VALUES, class KeyT>
+template<bool IDENTITY_VALUES, class KeyT, unsigned int ITEMS>
 __global__ void __launch_bounds__(kBlock) onesweep_pass(const KeyT* __restrict__ keys_in,
                                                         const uint32_t* __restrict__ vals_in,
                                                         KeyT* __restrict__ keys_out,
@@ -193,8 +203,12 @@ __global__ void __launch_bounds__(kBlock) onesweep_pass(const KeyT* __restrict__
                                                         uint32_t* __restrict__ status,
                                                         uint32_t* __restrict__ error)
     {
+    constexpr unsigned int kTile = kBlock * ITEMS;
+    // keys, then values, in digit order: in turn in the same words (12 items and 64-bit keys: two
+    // workgroups fit a CU instead of one, a pass over 2.1 10^6 keys 27 us instead of 31; more than two
+    // would need fewer registers than 12 items take: 64 or 80 registers spill, 10 to 14% slower builds)
     __shared__ KeyT s_keys[kTile];
-    __shared__ uint32_t s_vals[kTile];
+    uint32_t* const s_vals = reinterpret_cast<uint32_t*>(s_keys);
     __shared__ uint32_t s_wave[kWaves][kRadix];
     __shared__ uint32_t s_tile_start[kRadix];
     __shared__ uint32_t s_dst[kRadix];
@@ -212,12 +226,12 @@ __global__ void __launch_bounds__(kBlock) onesweep_pass(const KeyT* __restrict__
     const uint32_t base = tile * kTile;
 
     // load (wave-striped); keys past the end carry digit 255 and sort last in the tile
-    KeyT k[kItems];
-    uint32_t v[kItems];
+    KeyT k[ITEMS];
+    uint32_t v[ITEMS];
     #pragma unroll
-    for (unsigned int i = 0; i < kItems; ++i)
+    for (unsigned int i = 0; i < ITEMS; ++i)
         {
-        const uint32_t idx = base + wave * (64 * kItems) + i * 64 + lane;
+        const uint32_t idx = base + wave * (64 * ITEMS) + i * 64 + lane;
         if (idx < n)
             {
             k[i] = keys_in[idx];
@@ -232,9 +246,9 @@ __global__ void __launch_bounds__(kBlock) onesweep_pass(const KeyT* __restrict__
 
     // rank inside the wave, item by item, lanes in order
     const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    uint32_t r[kItems];
+    uint32_t r[ITEMS];
     #pragma unroll
-    for (unsigned int i = 0; i < kItems; ++i)
+    for (unsigned int i = 0; i < ITEMS; ++i)
         {
         const uint32_t d = static_cast<uint32_t>(k[i] >> shift) & (kRadix - 1);
         uint64_t same = ~0ull;
@@ -288,25 +302,34 @@ __global__ void __launch_bounds__(kBlock) onesweep_pass(const KeyT* __restrict__
         uint32_t excl = 0;
         if (tile != 0)
             {
-            int32_t j = static_cast<int32_t>(tile) - 1;
-            while (j >= 0)
+            bool found = false;
+            for (int32_t j = static_cast<int32_t>(tile) - 1; !found; j -= static_cast<int32_t>(kWindow))
                 {
+                // kWindow tiles' words in flight (short tiles look back over three times as many);
+                // before tile 0 lies a prefix of nothing
                 const uint32_t* w = status + static_cast<size_t>(j) * kRadix + d;
-                uint32_t s = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                uint32_t spins = 0;
-                while ((s >> 30) == 0u)
+                uint32_t s[kWindow];
+                #pragma unroll
+                for (int32_t i = 0; i < static_cast<int32_t>(kWindow); ++i)
+                    s[i] = j >= i ? __hip_atomic_load(w - i * static_cast<int32_t>(kRadix), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : kFlagPrefix;
+                #pragma unroll
+                for (int32_t i = 0; i < static_cast<int32_t>(kWindow); ++i)
                     {
-                    if (++spins > kSpinLimit)
+                    if (found) continue;
+                    uint32_t spins = 0;
+                    while ((s[i] >> 30) == 0u)
                         {
-                        atomicOr(error, 1u);
-                        break;
+                        if (++spins > kSpinLimit)
+                            {
+                            atomicOr(error, 1u);
+                            break;
+                            }
+                        __builtin_amdgcn_s_sleep(1);
+                        s[i] = __hip_atomic_load(w - i * static_cast<int32_t>(kRadix), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                         }
-                    __builtin_amdgcn_s_sleep(1);
-                    s = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    excl += s[i] & kValueMask;
+                    found = (s[i] >> 30) != 1u;     // inclusive prefix (or gave up)
                     }
-                excl += s & kValueMask;
-                if ((s >> 30) != 1u) break;     // inclusive prefix found (or gave up)
-                --j;
                 }
             __hip_atomic_store(my, kFlagPrefix | ((excl + tile_count) & kValueMask), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
@@ -314,29 +337,35 @@ __global__ void __launch_bounds__(kBlock) onesweep_pass(const KeyT* __restrict__
     }
     __syncthreads();
 
-    // scatter into LDS in digit order
+    // scatter into LDS in digit order, and contiguous runs per digit to global memory: keys, then
+    // values
+    const uint32_t nvalid = (n - base < kTile) ? (n - base) : kTile;
     #pragma unroll
-    for (unsigned int i = 0; i < kItems; ++i)
+    for (unsigned int i = 0; i < ITEMS; ++i)
         {
         const uint32_t d = static_cast<uint32_t>(k[i] >> shift) & (kRadix - 1);
-        const uint32_t pos = s_tile_start[d] + s_wave[wave][d] + r[i];
-        s_keys[pos] = k[i];
-        s_vals[pos] = v[i];
+        r[i] += s_tile_start[d] + s_wave[wave][d];
+        s_keys[r[i]] = k[i];
         }
     __syncthreads();
-
-    // contiguous runs per digit to global memory
-    const uint32_t nvalid = (n - base < kTile) ? (n - base) : kTile;
-    for (uint32_t j = tid; j < nvalid; j += kBlock)
+    uint32_t to[ITEMS];
+    #pragma unroll
+    for (unsigned int i = 0; i < ITEMS; ++i)
         {
+        const uint32_t j = i * kBlock + tid;
         const KeyT key = s_keys[j];
-        const uint32_t dst = s_dst[static_cast<uint32_t>(key >> shift) & (kRadix - 1)] + j;
-        if (dst < n)       // always true unless a look-back gave up (error flag set)
-            {
-            keys_out[dst] = key;
-            vals_out[dst] = s_vals[j];
-            }
+        to[i] = s_dst[static_cast<uint32_t>(key >> shift) & (kRadix - 1)] + j;
+        // dst < n always, unless a look-back gave up (error flag set)
+        if (j >= nvalid || to[i] >= n) to[i] = ~0u;
+        else keys_out[to[i]] = key;
         }
+    __syncthreads();
+    #pragma unroll
+    for (unsigned int i = 0; i < ITEMS; ++i) s_vals[r[i]] = v[i];
+    __syncthreads();
+    #pragma unroll
+    for (unsigned int i = 0; i < ITEMS; ++i)
+        if (to[i] != ~0u) vals_out[to[i]] = s_vals[i * kBlock + tid];
     }
 
 constexpr unsigned int kSmallBlock = 1024;
@@ -525,14 +554,17 @@ inline bool sort_passes(KeyT* keys, uint32_t* vals, KeyT* keys_alt, uint32_t* va
         KeyT* ko = alt ? keys : keys_alt;
         uint32_t* vo = alt ? vals : vals_alt;
         uint32_t* st = ws.status + static_cast<size_t>(p) * ws.tiles * kRadix;
-        if (p == 0 && identity_values)
-            hipLaunchKernelGGL((kernel::onesweep_pass<true, KeyT>), dim3(ws.tiles), dim3(kBlock), 0, stream,
-                               ki, vi, ko, vo, n, p * kBits, ws.hist + p * kRadix, ws.passes * kRadix, ws.tile_counter + p, st,
+        const auto launch = [&](auto identity, auto items) {
+            hipLaunchKernelGGL((kernel::onesweep_pass<decltype(identity)::value, KeyT, decltype(items)::value>), dim3(ws.tiles), dim3(kBlock),
+                               0, stream, ki, vi, ko, vo, n, p * kBits, ws.hist + p * kRadix, ws.passes * kRadix, ws.tile_counter + p, st,
                                ws.error);
-        else
-            hipLaunchKernelGGL((kernel::onesweep_pass<false, KeyT>), dim3(ws.tiles), dim3(kBlock), 0, stream,
-                               ki, vi, ko, vo, n, p * kBits, ws.hist + p * kRadix, ws.passes * kRadix, ws.tile_counter + p, st,
-                               ws.error);
+        };
+        const auto launch_items = [&](auto identity) {
+            if (n <= kShortKeys) launch(identity, std::integral_constant<unsigned int, kShortItems>());
+            else launch(identity, std::integral_constant<unsigned int, kItems>());
+        };
+        if (p == 0 && identity_values) launch_items(std::true_type());
+        else launch_items(std::false_type());
         alt = !alt;
         }
     check_launch("radix sort pass");

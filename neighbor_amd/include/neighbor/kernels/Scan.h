@@ -1,9 +1,11 @@
 // Scan.h -- exclusive scan of u32 counts into u64 offsets (CSR row starts), in index order
 // or in the order of a permutation (rows laid out in traversal order).
 //
-// Three launches, no inter-block waiting: per-tile sums, a one-block scan of the
-// tile sums, then per-tile scans offset by their tile's start.  Tile = 256 threads x
-// 8 counts.  offsets has n+1 entries; offsets[n] is the total.
+// Two launches, no inter-block waiting: per-tile sums, then per-tile scans, each offset by the sum
+// of the tiles before it, which its own block adds up (up to kAddedTiles tiles; with more of them
+// a one-block scan of the tile sums runs in between: a launch of 5 us, against the reads of at
+// most kAddedTiles sums per block from L2).  Tile = 256 threads x 8 counts.  offsets has n+1
+// entries; offsets[n] is the total.
 #ifndef NEIGHBOR_KERNELS_SCAN_H_
 #define NEIGHBOR_KERNELS_SCAN_H_
 
@@ -20,6 +22,7 @@ namespace scan
 constexpr unsigned int kBlock = 256;
 constexpr unsigned int kItems = 8;
 constexpr unsigned int kTile = kBlock * kItems;
+constexpr unsigned int kAddedTiles = 2048;
 
 inline unsigned int num_tiles(uint32_t n) { return (n + kTile - 1) / kTile; }
 inline size_t scratch_bytes(uint32_t n) { return (static_cast<size_t>(num_tiles(n)) + 1) * sizeof(unsigned long long); }
@@ -85,6 +88,8 @@ __global__ void __launch_bounds__(1024) scan_sums(unsigned long long* __restrict
     if (threadIdx.x == 0) sums[m] = carry;
     }
 
+//! SCANNED: sums holds the scan of the tile sums (and the total), else the sums themselves.
+template<bool SCANNED>
 __global__ void __launch_bounds__(kBlock) tile_scan(const uint32_t* __restrict__ counts, const uint32_t* __restrict__ perm,
                                                     uint32_t n, const unsigned long long* __restrict__ sums,
                                                     unsigned long long* __restrict__ offsets)
@@ -99,14 +104,23 @@ __global__ void __launch_bounds__(kBlock) tile_scan(const uint32_t* __restrict__
         c[i] = (base + i < n) ? count_at(counts, perm, base + i) : 0u;
         s += c[i];
         }
-    unsigned long long run = sums[blockIdx.x] + block_exclusive(s, s_tmp, nullptr);
+    unsigned long long own, run;
+    if constexpr (SCANNED) run = sums[blockIdx.x] + block_exclusive(s, s_tmp, &own);
+    else
+        {
+        unsigned long long before = 0ull, base_sum;
+        for (unsigned int j = threadIdx.x; j < blockIdx.x; j += kBlock) before += sums[j];
+        (void)block_exclusive(before, s_tmp, &base_sum);
+        run = base_sum + block_exclusive(s, s_tmp, &own);
+        own += base_sum;
+        }
     #pragma unroll
     for (unsigned int i = 0; i < kItems; ++i)
         {
         if (base + i < n) offsets[perm ? perm[base + i] : base + i] = run;
         run += c[i];
         }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) offsets[n] = sums[gridDim.x];
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) offsets[n] = SCANNED ? sums[gridDim.x] : own;
     }
 //! Exclusive scan of n <= kGroupScanMax u64 values in one block, in rounds of 1024 coalesced
 //! values (the loads of all rounds issued first), offset by *carry when carry is given (read
@@ -184,8 +198,15 @@ inline void exclusive_scan(const uint32_t* counts, uint32_t n, unsigned long lon
         return;
         }
     hipLaunchKernelGGL(kernel::tile_sums, dim3(tiles), dim3(kBlock), 0, stream, counts, perm, n, sums);
-    hipLaunchKernelGGL(kernel::scan_sums, dim3(1), dim3(1024), 0, stream, sums, tiles);
-    hipLaunchKernelGGL(kernel::tile_scan, dim3(tiles), dim3(kBlock), 0, stream, counts, perm, n, sums, offsets);
+    if (tiles <= kAddedTiles)
+        {
+        hipLaunchKernelGGL(kernel::tile_scan<false>, dim3(tiles), dim3(kBlock), 0, stream, counts, perm, n, sums, offsets);
+        }
+    else
+        {
+        hipLaunchKernelGGL(kernel::scan_sums, dim3(1), dim3(1024), 0, stream, sums, tiles);
+        hipLaunchKernelGGL(kernel::tile_scan<true>, dim3(tiles), dim3(kBlock), 0, stream, counts, perm, n, sums, offsets);
+        }
     check_launch("exclusive_scan");
     }
 
