@@ -35,7 +35,7 @@ namespace neighbor
 //! Traversal variant of the batched walk.
 enum class BatchVariant
     {
-    Wave = 0,   //!< one rope path per wave of 64 Morton-consecutive queries (wave::walk)
+    Wave = 0,   //!< node fronts for 64 Morton-consecutive queries per wave (front::walk)
     Lane = 1    //!< one rope path per lane
     };
 

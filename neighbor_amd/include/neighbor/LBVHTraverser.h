@@ -351,10 +351,9 @@ class LBVHTraverser : public Tunable<unsigned int>
                         {
                         if (m_visit_words < visitLogWords(query.size()))
                             throw std::invalid_argument("the visit log holds fewer words than the traversal's waves write");
-                        hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_wave<OutputOpT, QueryOpT, TranslateOpT, TransformOpT, true>),
-                                           grid, dim3(256), 0, params.stream, out, m_float.get(), lbvh.getSortedPoints().get(),
-                                           lbvh.getPrimitives().get(), m_lbvh_lo.get(), m_lbvh_hi.get(), m_root, query, images,
-                                           transform, order, lbvh.getNNodes(), m_visits);
+                        hipLaunchKernelGGL((gpu::kernel::lbvh_visit_log<QueryOpT, TranslateOpT>), grid, dim3(256), 0, params.stream,
+                                           out, m_float.get(), lbvh.getSortedPoints().get(), m_lbvh_lo.get(), m_lbvh_hi.get(), m_root,
+                                           query, images, order, lbvh.getNNodes(), m_visits);
                         return;
                         }
                     else

@@ -54,7 +54,7 @@ constexpr unsigned int kSmallTree = 60000;
 constexpr unsigned int kTeam = 4;           //!< waves of a team (one block)
 
 //! Magnitude up to which coordinates, radii and image vectors take this walk (others, and
-//! infinities and NaN, take wave::walk): squares and their sums stay finite in float.
+//! infinities and NaN, take lane_walk): squares and their sums stay finite in float.
 constexpr float kMaxCoordinate = 0x1p46f;
 //! Leaves whose squared distance from the wave's origin is not below this are out of every
 //! query's reach (at most (sqrt(3) 2 + 1) 2^46 < 10^15 away).
