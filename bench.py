@@ -276,7 +276,7 @@ def main():
     build_gbs = BUILD_BYTES_PER_PRIM * N / (build_total_ms * 1e-3) / 1e9
     traffic, traffic_note = profiled_traffic(dominant)
 
-    # wave-walk statistics of one untimed count pass (per-wave visit log)
+    # statistics of a walk by single rope paths: one untimed count pass with the visit log
     walk_stats = None
     if args.variant in (nb.NB_VARIANT_WAVE, nb.NB_VARIANT_WAVE_QUANTIZED):
         vlog = torch.zeros(nb.LBVHTraverser.visit_log_words(N), dtype=torch.int32, device="cuda")
@@ -285,13 +285,11 @@ def main():
         torch.cuda.synchronize()
         tr.set_visit_log(None)
         v = vlog.view(-1, 3).to(torch.int64).sum(dim=0).tolist()
-        cnt_s = stage_two["count"] * 1e-3
         walk_stats = {"wave_node_records_loaded": v[0], "wave_bucket_visits": v[1], "wave_bucket_leaves": v[2],
                       "node_tests_per_query": v[0] * 64 / N, "leaf_tests_per_query": v[2] * 64 / N,
                       "bucket_visits_per_wave": v[1] / ((N + 63) // 64),
-                      "node_records_per_s_count": v[0] / cnt_s, "node_tests_per_s_count": v[0] * 64 / cnt_s,
-                      "note": "a wave loads each visited node record once for its 64 queries (node and leaf "
-                              "tests count 64 lanes each); rates over the count stage time"}
+                      "note": "one rope path per wave of 64 queries over the same records (node and leaf tests "
+                              "count 64 lanes each); the timed walks go by node fronts"}
 
     result = {
         "metric": "exact neighbor pairs/s (N=1M uniform rho=0.85 r=2.8, 27 images; full LBVH build + neighbor "
@@ -602,7 +600,6 @@ def cpu_baseline_leg(args, np, pts, sph, L, lo, hi, total_pairs, result):
     for var in ("variant0", "variant1"):
         if var in ref_sem:
             ref_sem[var]["node_visits_per_query"] = rr["visits"] / sample
-            ref_sem[var]["node_visits_per_s_count"] = rr["visits"] / sample * N / (ref_sem[var]["count_ms"] * 1e-3)
     lbvh_step = t_build + per_query * N
     return {
         "value": total_pairs / t_all, "unit": "pairs/s", "cores": threads, "kind": "port",

@@ -40,8 +40,8 @@ extern "C" {
 #define NB_VARIANT_QUANTIZED 0        /* 16-B quantized rope records (the reference's traverser) */
 #define NB_VARIANT_FLOAT_ROPE 1       /* 32-B records of decoded quantized boxes: same results, no decode work */
 #define NB_VARIANT_FLOAT_ROPE_EXACT 2 /* 32-B records of exact node boxes: for the exact queries */
-#define NB_VARIANT_WAVE 3             /* exact queries only: one rope path per wave of 64 queries, bucket leaves */
-#define NB_VARIANT_WAVE_QUANTIZED 4   /* the wave walk over decoded quantized boxes: reference results, any query */
+#define NB_VARIANT_WAVE 3             /* exact queries only: 32-B records of exact boxes, bucket leaves */
+#define NB_VARIANT_WAVE_QUANTIZED 4   /* the same over decoded quantized boxes: reference results, any query */
 
 typedef struct nb_lbvh nb_lbvh;
 typedef struct nb_traverser nb_traverser;
@@ -122,11 +122,11 @@ int nb_traverser_set_variant(nb_traverser* trav, int variant);
  * setup.  (No reference counterpart.) */
 int nb_traverser_set_bucket_size(nb_traverser* trav, uint32_t bucket);
 
-/* Launch shape of the exact wave walks (nb_traverse_exact_count / _pairs / _rows /
- * _rows_placed): per XCD, the last `groups` groups of 256 queries run as `split` blocks (1, 2
- * or 4) of 256/split queries each, so the waves that start last in the launch are shorter.
- * Default 32 groups, split 2 (the last wave of each SIMD of an XCD); groups = 0: one block per
- * group.  Results do not depend on it.  (No reference counterpart.) */
+/* Launch shape of traversals of more than 65,536 queries (nb_traverse_*; not _rows_placed, whose
+ * blocks serve whole groups): per XCD, the last `groups` groups of 256 queries run as `split`
+ * blocks (1, 2 or 4) of 256/split queries each, so the waves that start last in the launch are
+ * shorter.  Default 32 groups (16 above 2^19 queries), split 2; groups = 0: one block per group.
+ * Results do not depend on it.  (No reference counterpart.) */
 int nb_traverser_set_tail_split(nb_traverser* trav, uint32_t groups, uint32_t split);
 
 /* Floats per record of the `points` argument of the exact calls (nb_traverse_exact_*): 3
@@ -135,7 +135,8 @@ int nb_traverser_set_tail_split(nb_traverser* trav, uint32_t groups, uint32_t sp
 int nb_traverser_set_point_stride(nb_traverser* trav, uint32_t stride);
 
 /* No counterpart in the reference (walk statistics of the wave variants, for measurement):
- * while set, every wave-variant count traversal through trav writes, per launched wave w, the
+ * while set, every wave-variant count traversal through trav takes one rope path per wave of 64
+ * queries (not the walk by node fronts) and writes, per launched wave w, the
  * node records it loaded, the buckets whose leaves it tested and the leaves in them to
  * log[3w .. 3w+2] (device memory of `words` u32; nb_visit_log_words(n) for n queries).  A
  * traversal whose waves need more words, or a wave traversal with another output op, fails

@@ -223,9 +223,9 @@ class LBVHTraverser:
         call("nb_traverser_set_bucket_size", self._h, int(bucket))
 
     def set_tail_split(self, groups: int, split: int = 2) -> None:
-        """Launch shape of the exact wave walks: per XCD, the last `groups` groups of 256
-        queries run as `split` (1, 2 or 4) smaller blocks (default 32, 2); groups 0 = one block
-        per group.  Results do not depend on it."""
+        """Launch shape of traversals of more than 65,536 queries: per XCD, the last `groups` groups
+        of 256 queries run as `split` (1, 2 or 4) smaller blocks (default 32, or 16 above 2^19
+        queries, and 2); groups 0 = one block per group.  Results do not depend on it."""
         call("nb_traverser_set_tail_split", self._h, int(groups), int(split))
 
     @staticmethod
@@ -234,8 +234,8 @@ class LBVHTraverser:
         return int(lib().nb_visit_log_words(int(n_queries)))
 
     def set_visit_log(self, log: Optional[torch.Tensor]) -> None:
-        """Wave-walk statistics (nb_traverser_set_visit_log): while set, each wave-variant count
-        traversal writes per launched wave (node records loaded, buckets tested, leaves in them)
+        """Walk statistics (nb_traverser_set_visit_log): while set, each wave-variant count
+        traversal takes one rope path per wave of 64 queries and writes per launched wave (node records loaded, buckets tested, leaves in them)
         into log (int32 device tensor, visit_log_words(n) entries or more); other wave traversals
         are refused meanwhile; None switches it off."""
         self._visit_log = log

@@ -12,8 +12,8 @@
 // ExactSphereQueryOp (with the float SphereQueryOp it reports fewer, tighter hits than the
 // reference); Wave (ExactSphereQueryOp only) exact-box records with bucket leaves; WaveQuantized
 // the same over decoded quantized boxes, for SphereQueryOp (results identical to Quantized) and
-// ExactSphereQueryOp.  Both queries walk by node fronts (kernels/FrontWalk.h) in every variant;
-// other query ops (rope variants) take one rope path per query.
+// ExactSphereQueryOp.  Both queries walk by node fronts (kernels/FrontWalk.h); other query ops, and
+// many exact queries over rope records (kRopeFronts), take one rope path per query.
 #ifndef NEIGHBOR_LBVH_TRAVERSER_H_
 #define NEIGHBOR_LBVH_TRAVERSER_H_
 
@@ -331,6 +331,53 @@ class LBVHTraverser : public Tunable<unsigned int>
                                n_nodes, tail, m_tail_split);
             }
 
+        //! Rope and quantized records by node fronts; false: not this query op, or too many exact queries.
+        template<class QueryOpT, class OutputOpT, class TranslateOpT>
+        bool traverse_rope_fronts(const LaunchParameters& params, const LBVH& lbvh, const QueryOpT& query, const OutputOpT& out,
+                                  const TranslateOpT& images, const unsigned int* order)
+            {
+            constexpr bool exact = std::is_same<QueryOpT, ExactSphereQueryOp>::value;
+            constexpr bool reference = std::is_same<QueryOpT, SphereQueryOp>::value;
+            if constexpr (exact || reference)
+                {
+                if (exact && query.size() > kRopeFronts) return false;
+                if (m_variant == TraversalVariant::Quantized)
+                    launch_front(params, query, out, images, order, lbvh.getNNodes(),
+                                 gpu::kernel::front::QuantizedSource{m_data.get(), float3(), float3(), float3(), lbvh.getNInternal()});
+                else
+                    launch_front(params, query, out, images, order, lbvh.getNNodes(),
+                                 gpu::kernel::front::RopeSource{m_float.get(), lbvh.getNInternal()});
+                return true;
+                }
+            return false;
+            }
+
+        //! One rope path per query: other query ops, and more exact queries than kRopeFronts.
+        template<class QueryOpT, class OutputOpT, class TranslateOpT>
+        void traverse_rope_paths(const LaunchParameters& params, const LBVH& lbvh, const QueryOpT& query, const OutputOpT& out,
+                                 const TranslateOpT& images, const unsigned int* order)
+            {
+            if constexpr (!std::is_same<QueryOpT, SphereQueryOp>::value)
+                {
+                const unsigned int block = checkParameter(params);
+                const dim3 grid(div_up(query.size(), block));
+                if (m_variant == TraversalVariant::Quantized)
+                    {
+                    hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_ropes<OutputOpT, QueryOpT, TranslateOpT>), grid, dim3(block), 0,
+                                       params.stream, out, data(), query, images, order, lbvh.getNNodes());
+                    }
+                else
+                    {
+                    LBVHFloatRopeData f;
+                    f.root = m_root;
+                    f.data = m_float.get();
+                    // the image bits use the unquantized root box stored by the compression
+                    hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_float_ropes<OutputOpT, QueryOpT, TranslateOpT>), grid, dim3(block), 0,
+                                       params.stream, out, f, m_lbvh_lo.get(), m_lbvh_hi.get(), query, images, order, lbvh.getNNodes());
+                    }
+                }
+            }
+
         //! Wave walk: defined for ExactSphereQueryOp only.
         template<class QueryOpT, class OutputOpT, class TranslateOpT, class TransformOpT>
         void traverse_wave(const LaunchParameters& params, const LBVH& lbvh, const QueryOpT& query, const OutputOpT& out,
@@ -377,6 +424,11 @@ class LBVHTraverser : public Tunable<unsigned int>
         //! images: 256 queries 44 us and 44, 512 71 and 54, 1000 89 and 44; without images 14 and 24,
         //! 21 and 30, 34 and 33; 10^6 (one rope path per lane) 8.2 ms and 0.7.
         static constexpr unsigned int kSortQueries = 256;
+        //! Exact queries over rope records up to which they walk by fronts.  These records are the choice
+        //! for few neighbors per query, where a walk is one short path down from the root: by fronts and
+        //! by a path per lane, 99,000 queries of 4 neighbors 75 and 100 us, 396,000 157 and 167, 990,000
+        //! 322 and 267 (1000 to 10,000 large ones in the same trees 50 to 151 and 229 to 395).
+        static constexpr unsigned int kRopeFronts = 1u << 18;
         //! Queries up to which four waves serve 64, 32, 16 or 4 queries together: one wave's chain of
         //! steps takes longer than the chip needs for all of them.  Exact count and fill of 10,000
         //! points (27 images): 82 and 115 us with a wave per 64 queries, 48 and 61 with teams for
@@ -466,42 +518,19 @@ void LBVHTraverser::traverse(const LaunchParameters& params, const LBVH& lbvh, c
     if (lbvh.getN() == 0) return;
     if (query.size() == 0 || images.size() == 0) return;
     if (images.size() > 32) throw image_limit_error();
-    const unsigned int block = checkParameter(params);
+    (void)checkParameter(params);
     if (!m_replay) compress(params, lbvh, transform);
 
     const unsigned int* order = (m_order && m_order_n == query.size()) ? m_order : nullptr;
-    const dim3 grid(div_up(query.size(), block));
     if (m_variant == TraversalVariant::Wave || m_variant == TraversalVariant::WaveQuantized)
         {
         traverse_wave(params, lbvh, query, out, images, transform, order);
         }
-    else if constexpr (placed)
-        {
-        // refused above
-        }
-    else if constexpr (std::is_same<QueryOpT, SphereQueryOp>::value || std::is_same<QueryOpT, ExactSphereQueryOp>::value)
-        {
-        if (m_variant == TraversalVariant::Quantized)
-            launch_front(params, query, out, images, order, lbvh.getNNodes(),
-                         gpu::kernel::front::QuantizedSource{m_data.get(), float3(), float3(), float3(), lbvh.getNInternal()});
-        else
-            launch_front(params, query, out, images, order, lbvh.getNNodes(),
-                         gpu::kernel::front::RopeSource{m_float.get(), lbvh.getNInternal()});
-        }
-    else if (m_variant == TraversalVariant::Quantized)
-        {
-        hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_ropes<OutputOpT, QueryOpT, TranslateOpT>), grid, dim3(block), 0,
-                           params.stream, out, data(), query, images, order, lbvh.getNNodes());
-        }
     else
         {
-        LBVHFloatRopeData f;
-        f.root = m_root;
-        f.data = m_float.get();
-        // the image bits use the unquantized root box stored by the compression
-        hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_float_ropes<OutputOpT, QueryOpT, TranslateOpT>), grid, dim3(block), 0,
-                           params.stream, out, f, m_lbvh_lo.get(), m_lbvh_hi.get(), query, images, order,
-                           lbvh.getNNodes());
+        // refused above: placed rows
+        if constexpr (!placed)
+            if (!traverse_rope_fronts(params, lbvh, query, out, images, order)) traverse_rope_paths(params, lbvh, query, out, images, order);
         }
     check_launch("lbvh_traverse");
     }

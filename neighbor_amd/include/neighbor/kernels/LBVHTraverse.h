@@ -372,7 +372,7 @@ __device__ __forceinline__ unsigned int xcd_block(unsigned int b, unsigned int G
     return x * q + (x < r ? x : r) + j;
     }
 
-//! Queries of one 256-thread block of the compacted walks (tail-split launch map).
+//! Queries of one 256-thread block (tail-split launch map).
 struct BlockSpan
     {
     unsigned int first;      //!< first query position of the block

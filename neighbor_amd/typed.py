@@ -10,9 +10,8 @@ indices of its type, as the reference requires: ``LBVHTraverser.h:366-390``, the
 at setup and traversal).  Particle i's row holds its hits in tree 0, then tree 1, ...; rows are
 laid out per query type, each type in its tree's Morton order.
 
-Each (query type, tree type) pair has its own best traversal: few neighbors per query (small
-radii, or sparse queries over a dense tree) favour one lane per query (float-rope records),
-many favour the wave walk over leaf buckets.  ``tune`` times the candidates on the current
+Each (query type, tree type) pair has its own best records: rope records, whose runs of up to 32
+leaves follow the tree, or bucket records of a size that suits the pair's neighbors.  ``tune`` times the candidates on the current
 configuration and keeps the fastest per pair; every candidate gives the same pairs.
 """
 from __future__ import annotations

@@ -293,3 +293,21 @@ def test_exact_query_other_points(nb, n):
         got = host(tr.exact_count(lb, torch.from_numpy(sph).cuda(), torch.from_numpy(other).cuda())).astype(np.int64)
         most = (near & (gap <= R + more)).sum(1)
         assert (got >= least).all() and (got <= most).all()
+
+
+@pytest.mark.parametrize("n", [262144, 262145])
+def test_exact_query_rope_records_by_size(nb, n):
+    """Both sides of the size from which exact queries over rope records take a path each: the counts
+    of the bucket records' walk."""
+    import torch
+    rng = np.random.default_rng(n)
+    pts, L = points_of(n, rng, "uniform")
+    d_pts = torch.from_numpy(pts).cuda()
+    sph = torch.cat([d_pts, torch.full((n, 1), 1.1, device="cuda")], 1).contiguous()
+    lb = nb.LBVH()
+    lb.build(d_pts, [0, 0, 0], [L] * 3)
+    order = lb.device_pointers()["primitive"]
+    want = nb.LBVHTraverser(variant=nb.NB_VARIANT_WAVE).exact_count(lb, sph, d_pts, order=order)
+    for variant in (nb.NB_VARIANT_QUANTIZED, nb.NB_VARIANT_FLOAT_ROPE, nb.NB_VARIANT_FLOAT_ROPE_EXACT):
+        got = nb.LBVHTraverser(variant=variant).exact_count(lb, sph, d_pts, order=order)
+        assert torch.equal(got, want)
