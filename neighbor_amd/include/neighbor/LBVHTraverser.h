@@ -322,7 +322,7 @@ class LBVHTraverser : public Tunable<unsigned int>
                     }
             // tail-split map (wave::tail_block): XCD 0 holds the most groups; the other XCDs'
             // blocks past their own count exit at once
-            const unsigned int tail = placed ? 0u : m_tail_set || n <= kShortTail ? m_tail_groups : kShortTailGroups;
+            const unsigned int tail = placed ? 0u : m_tail_set || (n > kAllSplit && n <= kHalfSplit) ? m_tail_groups : n <= kAllSplit ? kAllSplitGroups : kTailGroups;
             const unsigned int G = div_up(n, 256);
             const unsigned int x0 = G / 8u + (G % 8u ? 1u : 0u);
             const dim3 grid = tail ? dim3(8u * (x0 + (m_tail_split - 1u) * std::min(x0, tail))) : dim3(G);
@@ -436,16 +436,19 @@ class LBVHTraverser : public Tunable<unsigned int>
         //! for 16 and for 4: 1000 points 35 and 47 us, 29 and 38; 4000 points 56 and 72, 45 and 56;
         //! 8000 points 48 and 65, 62 and 77.
         static constexpr unsigned int kTeamQueries = 1u << 16;
-        //! Tail split (wave::tail_block): per XCD, the last m_tail_groups groups of 256 queries run
-        //! as m_tail_split blocks each, so that the waves that start last are shorter.  Exact count
-        //! and fill of 300,007 points: 204 and 297 us with 32 groups, 222 and 329 with none; of 10^6
-        //! points, where the tail is a smaller part, 348 and 581 us with 16 groups, 358 and 597 with
-        //! 32, 356 and 594 with none.
+        //! Tail split (wave::tail_block): per XCD, the last groups of 256 queries run as m_tail_split
+        //! blocks each, so that the waves that start last are shorter.  Up to kAllSplit queries, which
+        //! leave wave slots free, all groups do (64 per XCD), up to kHalfSplit 32 of each XCD, above it
+        //! 16.  Exact count and fill in us with 0, 16, 32 and 64 groups (27 images): 100,000 points
+        //! 89/136, 76/116, 72/113 and 73/116; 131,071 92/140, 87/138, 82/131 and 81/125; 200,000
+        //! 148/214, 119/180, 145/225 and 143/232; 300,007 212/322, 206/287, 206/293 and 207/304; 500,000
+        //! 257/374, 236/359, 247/377 and 253/385; 10^6 with 0, 16 and 32 356/594, 348/581 and 358/597.
+        //! Without images: 70,000 points 70/94, 62/84, 59/83 and 54/76; 131,071 76/104, 74/106, 69/100
+        //! and 72/100.  16 groups in four blocks: 300,007 197/293, 500,000 233/355, 200,000 135/206.
         unsigned int m_tail_groups = 32;
         unsigned int m_tail_split = 2;
         bool m_tail_set = false;        //!< by setTailSplit: kept for any number of queries
-        static constexpr unsigned int kShortTail = 1u << 19;
-        static constexpr unsigned int kShortTailGroups = 16;
+        static constexpr unsigned int kAllSplit = 3u << 15, kAllSplitGroups = 64, kHalfSplit = 1u << 17, kTailGroups = 16;
 
     public:
         //! Leaves per bucket of the wave variant (1..64); takes effect at the next compression.
