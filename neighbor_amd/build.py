@@ -41,8 +41,10 @@ def build(verbose: bool = False) -> str:
 
 
 EXAMPLES = [os.path.join(HERE, "examples", "periodic_neighbors.hip"),
-            # device probe of the rounding helpers and bounding volumes, run by the GPU tests
-            os.path.join(ROOT, "tests", "device", "device_math.hip")]
+            # device probe of the rounding helpers and bounding volumes, and traversals with output ops
+            # of a program's own: run by the GPU tests
+            os.path.join(ROOT, "tests", "device", "device_math.hip"),
+            os.path.join(ROOT, "tests", "device", "custom_output.hip")]
 
 
 def build_examples(verbose: bool = False) -> list:

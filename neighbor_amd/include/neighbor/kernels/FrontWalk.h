@@ -19,6 +19,7 @@
 
 #include "LBVHTraverse.h"
 
+#include <new>
 #include <stdint.h>
 
 namespace neighbor
@@ -555,6 +556,17 @@ __device__ __forceinline__ void write_hits(unsigned int* __restrict__ neigh, uns
         }
     }
 
+//! The thread data of an output op.  A set-up runs once for each query, in a lane that serves it: an
+//! op of a program's own may clear or reserve there what it writes to later.
+template<class ThreadDataT>
+union Slot
+    {
+    char none;
+    ThreadDataT data;
+    __device__ Slot() : none(0) {}
+    __device__ ~Slot() {}
+    };
+
 //! The walk over the subtree of `root` (n_nodes nodes) for one query per lane, by one wave or, TEAM,
 //! by the four waves of a block for the same queries; false: not walked (queries too scattered).
 /*!
@@ -612,7 +624,10 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
     const unsigned int member = TEAM ? static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6))) : 0u;
     const unsigned int n_internal = src.n_internal;
     const unsigned int nimg = images.size() < 32u ? images.size() : 32u;
-    typename OutputOpT::ThreadData result = out.setup(idx, q);
+    Slot<typename OutputOpT::ThreadData> slot;
+    typename OutputOpT::ThreadData& result = slot.data;
+    // counts and rows only read in their set-ups: all lanes, before the loops (spills otherwise)
+    if constexpr (kCount || kRows) new (&slot.data) typename OutputOpT::ThreadData(out.setup(idx, q));
     const float r = fabsf(q.w);
 
     // image vectors in float and their largest component
@@ -680,6 +695,8 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
         // a team are still walked faster by its four waves than one per lane: 4000 spheres of
         // radius 5.9 in a tree of 396,000 points, 16 per team, 123 us against 185)
         if (pass == 0 && n_nodes > kSmallTree && (!TEAM || __popcll(actm) > 16) && 8u * static_cast<unsigned int>(__popcll(qwide)) > kScattered * static_cast<unsigned int>(__popcll(actm))) return false;
+        if constexpr (!kCount && !kRows)
+            if (pass == 0 && valid) new (&slot.data) typename OutputOpT::ThreadData(out.setup(idx, q));
         if (spread && qwide)
             {
             #pragma unroll
