@@ -79,9 +79,6 @@ struct NeighborListOp
 //! or past the buffer capacity are dropped and still counted (nneigh may be null).
 struct PairListOp
     {
-    //! The wave walk may stage hits in LDS and write them to neigh/image[pos, end) in runs.
-    static constexpr bool kStaged = true;
-
     PairListOp(const unsigned long long* offsets_, unsigned int* neigh_, unsigned char* image_, unsigned int* nneigh_,
                unsigned long long capacity_)
         : offsets(offsets_), neigh(neigh_), image(image_), nneigh(nneigh_), capacity(capacity_) {}
@@ -138,8 +135,6 @@ struct PairListOp
 //! spill[0] is the end of the used positions and spill[1] the number of moved rows.
 struct RowPairOp
     {
-    static constexpr bool kStaged = true;
-
     RowPairOp(unsigned long long* start_, unsigned int* limit_, unsigned int* neigh_, unsigned char* image_,
               unsigned int* nneigh_, unsigned long long capacity_, unsigned long long* spill_ = nullptr)
         : start(start_), limit(limit_), neigh(neigh_), image(image_), nneigh(nneigh_), capacity(capacity_), spill(spill_) {}

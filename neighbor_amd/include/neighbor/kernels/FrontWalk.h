@@ -456,11 +456,17 @@ __device__ __forceinline__ void batch_decide(const FrontWave& W, const float B[4
         }
     }
 
-//! Rows of an output op that the walk writes itself: pair rows (wave::staged), fixed-stride lists.
+//! Rows that the walk writes itself: the library's pair rows and fixed-stride lists.  Any other op,
+//! also one derived from these, gets its hits through process().
 template<class OutputOpT>
 struct Rows
     {
-    static constexpr bool kOn = wave::staged<OutputOpT>::value;
+    static constexpr bool kOn = false;
+    };
+template<class OutputOpT>
+struct PairRows
+    {
+    static constexpr bool kOn = true;
     typedef typename OutputOpT::ThreadData ThreadData;
     __device__ static __forceinline__ unsigned long long at(const OutputOpT&, const ThreadData& t) { return t.pos; }
     __device__ static __forceinline__ unsigned long long end(const OutputOpT&, const ThreadData& t) { return t.end; }
@@ -472,6 +478,9 @@ struct Rows
     __device__ static __forceinline__ unsigned int* neigh(const OutputOpT& o) { return o.neigh; }
     __device__ static __forceinline__ unsigned char* image(const OutputOpT& o) { return o.image; }
     };
+template<> struct Rows<PairListOp> : PairRows<PairListOp> {};
+template<> struct Rows<RowPairOp> : PairRows<RowPairOp> {};
+template<> struct Rows<PlacedRowPairOp> : PairRows<PlacedRowPairOp> {};
 template<>
 struct Rows<NeighborListOp>
     {
@@ -488,11 +497,6 @@ struct Rows<NeighborListOp>
     __device__ static __forceinline__ void add(ThreadData& t, const uint32_t n) { t.num_neigh += n; }
     __device__ static __forceinline__ unsigned int* neigh(const NeighborListOp& o) { return o.neigh_list; }
     __device__ static __forceinline__ unsigned char* image(const NeighborListOp&) { return nullptr; }
-    };
-template<>
-struct Rows<CountNeighborsOp>
-    {
-    static constexpr bool kOn = false;
     };
 
 //! Writes the hits (bit s: batch leaf s) of each lane's query at its row position: `at`, before

@@ -429,13 +429,6 @@ __device__ __forceinline__ float threshold(const ExactSphere& v) { return v.T; }
 __device__ __forceinline__ float3 center(const BoundingSphere& v) { return v.origin; }
 __device__ __forceinline__ float threshold(const BoundingSphere& v) { return approx::fmul_ru(v.Rsq, 1.0f + 0x1p-18f); }
 
-//! Pair output ops (kStaged): rows of pairs at positions their thread data holds (pos, end), which
-//! the walks write themselves.
-template<class O, class = void>
-struct staged : std::false_type {};
-template<class O>
-struct staged<O, typename std::enable_if<O::kStaged>::type> : std::true_type {};
-
 //! Output ops whose rows the wave kernels place before the walk (kPlacedRows: PlacedRowPairOp;
 //! every thread of the 256-thread block takes part).
 template<class O, class = void>

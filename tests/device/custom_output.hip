@@ -4,7 +4,9 @@
 // Usage: custom_output.bin MODE in out
 //   in : n, nq, variant, bucket, order (0 none, 1 the tree's, 2 given), nimg, exact (u32 each), the
 //        box side (float), points (n float3), spheres (nq float4), images (nimg double3), order (nq u32)
-//   out: per query, sums, set-ups and finalizes (mode log)
+//        and, mode half, the row starts (nq + 1 u64)
+//   out: per query, sums, set-ups and finalizes (mode log); counts of the hits kept, then the pairs
+//        (mode half)
 #include "neighbor/neighbor.h"
 
 #include <hip/hip_runtime.h>
@@ -44,6 +46,16 @@ struct LogOp
     unsigned int* finals;
     };
 
+// Pair rows of the hits whose primitive is not below the query's index.
+struct HalfPairsOp : public PairListOp
+    {
+    using PairListOp::PairListOp;
+    __device__ void process(ThreadData& t, const int primitive, const unsigned int image) const
+        {
+        if (static_cast<unsigned int>(primitive) >= t.idx) PairListOp::process(t, primitive, image);
+        }
+    };
+
 namespace
 {
 template<class T>
@@ -80,6 +92,7 @@ int run(const std::string& mode, const char* in, const char* out)
     const std::vector<float4> spheres = take<float4>(f, nq);
     const std::vector<double3> images = take<double3>(f, nimg);
     const std::vector<unsigned int> order = take<unsigned int>(f, head[4] == 2u ? nq : 0u);
+    const std::vector<unsigned long long> starts = take<unsigned long long>(f, mode == "half" ? nq + 1u : 0u);
     std::fclose(f);
     std::vector<float3> images_f;
     for (const double3& t : images)
@@ -115,6 +128,15 @@ int run(const std::string& mode, const char* in, const char* out)
         download(o, op.sums, nq);
         download(o, op.setups, nq);
         download(o, op.finals, nq);
+        }
+    else if (mode == "half")
+        {
+        const size_t total = starts[nq];
+        const HalfPairsOp op(upload(starts), upload(std::vector<unsigned int>(total, ~0u)), nullptr,
+                             upload(std::vector<unsigned int>(nq, 0u)), total);
+        traverse(op);
+        download(o, op.nneigh, nq);
+        download(o, op.neigh, total);
         }
     else throw std::runtime_error("unknown mode");
     std::fclose(o);

@@ -25,7 +25,7 @@ def orc():
     return oracle
 
 
-def run(mode, tmp_path, pts, sph, imgs, L, variant, order, exact, bucket=16):
+def run(mode, tmp_path, pts, sph, imgs, L, variant, order, exact, bucket=16, starts=None):
     head = np.array([len(pts), len(sph), variant, bucket, 2 if isinstance(order, np.ndarray) else order, len(imgs), int(exact)], np.uint32)
     src, dst = str(tmp_path / "in"), str(tmp_path / "out")
     with open(src, "wb") as f:
@@ -33,6 +33,8 @@ def run(mode, tmp_path, pts, sph, imgs, L, variant, order, exact, bucket=16):
             f.write(np.ascontiguousarray(a).tobytes())
         if isinstance(order, np.ndarray):
             f.write(order.astype(np.uint32).tobytes())
+        if starts is not None:
+            f.write(starts.astype(np.uint64).tobytes())
     r = subprocess.run([EXE, mode, src, dst], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stderr
     return np.fromfile(dst, np.uint32)
@@ -70,3 +72,26 @@ def test_set_up_once(orc, tmp_path, n, order, variant, exact):
     want = np.bincount(i, weights=31.0 * j + 7.0 * k + 1.0, minlength=n).astype(np.int64)
     assert (got[1] == 1).all() and (got[2] == 1).all()
     assert np.array_equal(got[0].astype(np.int64), want % (1 << 32))
+
+
+@pytest.mark.parametrize("variant,exact", [(QUANTIZED, False), (FLOAT_ROPE, True), (WAVE_QUANTIZED, False), (WAVE, True)])
+@pytest.mark.parametrize("n,order", [(50, 0), (2000, 0), (70001, 1)])
+def test_derived_rows(orc, tmp_path, n, order, variant, exact):
+    """An op derived from the library's pair rows that keeps some of the hits."""
+    from neighbor_amd.workloads import images27
+    log(f"derived pair rows: n={n} order={order} variant={variant} exact={exact}")
+    rng = np.random.default_rng(n + 1)
+    L = float(np.float32((n / 0.85) ** (1.0 / 3.0)))
+    pts = (rng.random((n, 3)) * L).astype(np.float32)
+    pts[pts >= np.float32(L)] = 0.0
+    sph = np.concatenate([pts, np.full((n, 1), 1.1)], 1).astype(np.float32)
+    imgs = images27(L, dtype=np.float64)
+    i, j, _ = hits(orc, pts, sph, imgs, L, exact)
+    keep = j >= i
+    counts = np.bincount(i[keep], minlength=n)
+    starts = np.concatenate([[0], np.cumsum(counts)])
+    got = run("half", tmp_path, pts, sph, imgs, L, variant, order, exact, starts=starts)
+    assert np.array_equal(got[:n].astype(np.int64), counts)
+    rows = np.repeat(np.arange(n), counts)
+    pairs = got[n:].astype(np.int64)
+    assert np.array_equal(pairs[np.lexsort((pairs, rows))], j[keep][np.lexsort((j[keep], i[keep]))])
