@@ -306,10 +306,19 @@ __device__ __forceinline__ void batch_traverse_body(const OutputOpT& out,
                 const Source src{nodes, points, primitive, NullTransformOp(), n_internal};
                 front::FrontWave& W = *reinterpret_cast<front::FrontWave*>(lds[wid]);
                 front::FrontPairs& P = *reinterpret_cast<front::FrontPairs*>(lds[wid] + sizeof(front::FrontWave));
-                const bool walked = !rooted || (front::takes<Source, QueryOpT>(valid, qd, images, root_box)
-                    && front::walk<false>(out, src, root, root_box, query, images, valid, idx, qd, 2u * nb - 1u, W, P, nullptr));
+                // as in lbvh_traverse_front
+                const bool fronts = rooted && front::takes<Source, QueryOpT>(images, root_box);
+                const unsigned long long mine = walk_kernels::wave::vote(valid && fronts && front::takes(qd));
+                unsigned long long alone = walk_kernels::wave::vote(valid && rooted) & ~mine;
+                if (mine && !front::walk<false>(out, src, root, root_box, query, images, walk_kernels::wave::lane_in(mine), idx, qd,
+                                                2u * nb - 1u, W, P, nullptr))
+                    alone |= mine;
                 if (valid && !rooted) out.finalize(out.setup(idx, qd));
-                else if (valid && !walked) front::lane_walk(out, src, root, stop, root_box, query, images, idx, qd, n_nodes);
+                else if (walk_kernels::wave::lane_in(alone))
+                    {
+                    const unsigned int i = primitive[s + it.first + lane];
+                    front::lane_walk(out, src, root, stop, root_box, query, images, i, query.setup(i), n_nodes);
+                    }
                 }
             }
         }

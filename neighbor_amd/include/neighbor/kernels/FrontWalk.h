@@ -1159,21 +1159,25 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
     return true;
     }
 
-//! True when every lane's query and every image vector (reference query, quantized boxes: and the
-//! root box, which holds every box) take the walk above (wave-uniform).
+__device__ __forceinline__ bool small(const float x, const float y, const float z)
+    {
+    return fabsf(x) < kMaxCoordinate && fabsf(y) < kMaxCoordinate && fabsf(z) < kMaxCoordinate;
+    }
+//! True when a query takes the walk above.
+__device__ __forceinline__ bool takes(const float4& q) { return small(q.x, q.y, q.z) && fabsf(q.w) < kMaxCoordinate; }
+
+//! True when the image vectors (reference query, quantized boxes: and the root box, which holds every
+//! box) let queries take the walk above (wave-uniform).
 template<class SrcT, class QueryOpT, class TranslateOpT>
-__device__ __forceinline__ bool takes(const bool valid, const float4& q, const TranslateOpT& images, const BoundingBox& root_box)
+__device__ __forceinline__ bool takes(const TranslateOpT& images, const BoundingBox& root_box)
     {
     const unsigned int lane = threadIdx.x & 63u;
     const unsigned int nimg = images.size() < 32u ? images.size() : 32u;
-    const auto small = [](const float x, const float y, const float z) {
-        return fabsf(x) < kMaxCoordinate && fabsf(y) < kMaxCoordinate && fabsf(z) < kMaxCoordinate;
-    };
-    bool ok = !valid || (small(q.x, q.y, q.z) && fabsf(q.w) < kMaxCoordinate);
+    bool ok = true;
     if (lane < nimg)
         {
         const double3 t = as_double3(images.get(lane));
-        ok = ok && small(static_cast<float>(t.x), static_cast<float>(t.y), static_cast<float>(t.z));
+        ok = small(static_cast<float>(t.x), static_cast<float>(t.y), static_cast<float>(t.z));
         }
     if constexpr (SrcT::kFirst || !std::is_same<QueryOpT, ExactSphereQueryOp>::value)
         ok = ok && small(root_box.lo.x, root_box.lo.y, root_box.lo.z) && small(root_box.hi.x, root_box.hi.y, root_box.hi.z);
@@ -1189,7 +1193,16 @@ __device__ __forceinline__ void lane_walk(const OutputOpT& out, const SrcT& src,
     {
     constexpr bool kExact = std::is_same<QueryOpT, ExactSphereQueryOp>::value;
     typename OutputOpT::ThreadData result = out.setup(idx, q);
-    const unsigned int nimg = images.size() < 32u ? images.size() : 32u;
+    unsigned int nimg = images.size() < 32u ? images.size() : 32u;
+    if constexpr (kExact)
+        {
+        // no distance from a center that is not finite is within a finite radius, and none within or from
+        // a NaN: not walked, where box tests let such centers through everywhere
+        const float inf = __builtin_huge_valf();
+        const bool finite = fabsf(q.x) < inf && fabsf(q.y) < inf && fabsf(q.z) < inf;
+        const bool within = finite ? q.w == q.w : fabsf(q.w) == inf && q.x == q.x && q.y == q.y && q.z == q.z;
+        if (!within) nimg = 0u;
+        }
     for (int pass = 0; pass < 2; ++pass)
         {
         for (unsigned int k = 0; k < nimg; ++k)
@@ -1337,10 +1350,18 @@ lbvh_traverse_front(const OutputOpT out,
     front::bind(src, root_box, bins);
     front::FrontWave& W = *reinterpret_cast<front::FrontWave*>(lds[wid]);
     front::FrontPairs& P = *reinterpret_cast<front::FrontPairs*>(lds[wid] + sizeof(front::FrontWave));
-    if (front::takes<SrcT, QueryOpT>(valid, q, images, root_box)
-        && front::walk<false>(out, src, root, root_box, query, images, valid, idx, q, n_nodes, W, P, nullptr)) return;
-    if (valid)
-        front::lane_walk(out, src, root, LBVHSentinel, root_box, query, images, idx, q, n_nodes);
+    // unusual queries take a path of their own after the others' walk (their lanes are kept as a mask and
+    // they are read again: nothing of them is held in registers meanwhile)
+    const bool fronts = front::takes<SrcT, QueryOpT>(images, root_box);
+    const unsigned long long mine = wave::vote(valid && fronts && front::takes(q));
+    unsigned long long alone = wave::vote(valid) & ~mine;
+    if (mine && !front::walk<false>(out, src, root, root_box, query, images, wave::lane_in(mine), idx, q, n_nodes, W, P, nullptr))
+        alone |= mine;
+    if (wave::lane_in(alone))
+        {
+        const unsigned int i = order ? order[t] : t;
+        front::lane_walk(out, src, root, LBVHSentinel, root_box, query, images, i, query.setup(i), n_nodes);
+        }
     }
 
 //! lbvh_traverse_front with the four waves of a block for the same `per` (4, 16, 32 or 64) queries:
@@ -1374,10 +1395,16 @@ lbvh_traverse_team(const OutputOpT out,
     front::bind(src, root_box, bins);
     front::FrontWave& W = *reinterpret_cast<front::FrontWave*>(lds[wid]);
     front::FrontPairs& P = *reinterpret_cast<front::FrontPairs*>(lds[wid] + sizeof(front::FrontWave));
-    if (front::takes<SrcT, QueryOpT>(valid, q, images, root_box)
-        && front::walk<true>(out, src, root, root_box, query, images, valid, idx, q, n_nodes, W, P, &team)) return;
-    if (valid && wid == 0u)
-        front::lane_walk(out, src, root, LBVHSentinel, root_box, query, images, idx, q, n_nodes);
+    const bool fronts = front::takes<SrcT, QueryOpT>(images, root_box);
+    const unsigned long long mine = wave::vote(valid && fronts && front::takes(q));
+    unsigned long long alone = wave::vote(valid) & ~mine;
+    if (mine && !front::walk<true>(out, src, root, root_box, query, images, wave::lane_in(mine), idx, q, n_nodes, W, P, &team))
+        alone |= mine;
+    if (wid == 0u && wave::lane_in(alone))
+        {
+        const unsigned int i = order ? order[t] : t;
+        front::lane_walk(out, src, root, LBVHSentinel, root_box, query, images, i, query.setup(i), n_nodes);
+        }
     }
 
 } // end namespace kernel

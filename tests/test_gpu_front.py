@@ -166,6 +166,55 @@ def test_unusual_queries(nb, orc, n):
             assert got[q] == want, (q, sph[q])
 
 
+@pytest.mark.parametrize("n", [40, 5000, 70000])
+@pytest.mark.parametrize("batched", [False, True])
+def test_unusual_queries_beside_rows(nb, n, batched):
+    """Exact rows of waves with a few unusual queries: the others' rows are those of a call without
+    them, NaN and infinite centers have no hits, a radius beyond the walk's range has every point."""
+    import torch
+    from neighbor_amd.api import exact_rows, exclusive_scan
+    from neighbor_amd.batch import LBVHBatch
+    rng = np.random.default_rng(n + 3)
+    pts, L = points_of(n, rng, "uniform")
+    plain = np.concatenate([pts, np.full((n, 1), 1.3, np.float32)], 1).astype(np.float32)
+    none, every = rng.choice(n, 8, replace=False).reshape(2, 4)
+    odd = plain.copy()
+    plain[none, :3] = -50.0 * L
+    odd[none[0], 0] = np.nan
+    odd[none[1], 3] = np.nan
+    odd[none[2], 1] = np.inf
+    odd[none[3], :3] = -np.inf
+    odd[every, 3] = (1e30, np.inf, -3e38, 1e15)
+    plain[every, 3] = 4.0 * L
+    d_pts = torch.from_numpy(pts).cuda()
+    box = torch.tensor([[0.0] * 3, [L] * 3], device="cuda")
+
+    def rows(sph):
+        d = torch.from_numpy(sph).cuda()
+        if batched:
+            b = LBVHBatch()
+            b.build(d_pts, torch.tensor([0, n], dtype=torch.int32, device="cuda"), box[:1].contiguous(), box[1:].contiguous())
+            b.setup()
+            counts = b.count(d, periodic=False)
+            start = exclusive_scan(counts)
+            return host(counts), host(start), host(b.pairs(d, start, periodic=False)[0])
+        lb = nb.LBVH()
+        lb.build(d_pts, [0, 0, 0], [L] * 3)
+        tr = nb.LBVHTraverser(variant=nb.NB_VARIANT_WAVE)
+        tr.setup(lb)
+        order = lb.device_pointers()["primitive"]
+        counts = tr.exact_count(lb, d, d_pts, order=order)
+        start = exclusive_scan(counts)
+        neigh = torch.full((int(start[-1]),), -1, dtype=torch.int32, device="cuda")
+        exact_rows(tr, lb, d, d_pts, start, counts, neigh, order=order)
+        return host(counts), host(start), host(neigh)
+
+    got, want = rows(odd), rows(plain)
+    assert (got[0][none] == 0).all() and (got[0][every] == n).all()
+    for g, w in zip(got, want):
+        assert np.array_equal(g, w)
+
+
 def test_two_streams_share_a_traverser(nb, orc):
     """Unordered queries (sorted on the device in the traverser's workspaces) on two streams and
     with other numbers of queries in turn."""
