@@ -41,10 +41,11 @@ def build(verbose: bool = False) -> str:
 
 
 EXAMPLES = [os.path.join(HERE, "examples", "periodic_neighbors.hip"),
-            # device probe of the rounding helpers and bounding volumes, and traversals with output ops
-            # of a program's own: run by the GPU tests
+            # device probe of the rounding helpers and bounding volumes, traversals with output ops of a
+            # program's own and from several threads: run by the GPU tests
             os.path.join(ROOT, "tests", "device", "device_math.hip"),
-            os.path.join(ROOT, "tests", "device", "custom_output.hip")]
+            os.path.join(ROOT, "tests", "device", "custom_output.hip"),
+            os.path.join(ROOT, "tests", "device", "shared_traverser.hip")]
 
 
 def build_examples(verbose: bool = False) -> list:

@@ -195,17 +195,19 @@ class LBVHTraverser : public Tunable<unsigned int>
         template<class TransformOpT>
         void compress(const LaunchParameters& params, const LBVH& lbvh, const TransformOpT& transform);
 
-        //! Workspace that sorts the queries of one launch: used by one stream at a time (done: the
-        //! last launch that reads it).
+        //! Workspace that sorts the queries of one launch (done: the last launch that reads it).
         struct QuerySort
             {
             shared_array<unsigned int> keys[2], vals[2], work;
             stream_t stream = nullptr;
             std::shared_ptr<void> done;     //!< hipEvent_t
             };
-        //! Bounded: a launch finds its stream's workspace, a free one, or waits for the oldest.  The
-        //! lock is held from the sort to the record of `done` (several threads may traverse at
-        //! once); a copy of the traverser starts with none.
+        //! Bounded: a launch takes the workspace last used with its stream's handle, a free one, a new
+        //! one or the oldest, and waits on the device for the workspace's last launch: equal handles
+        //! may be different streams (each thread's hipStreamPerThread, a new stream at a destroyed
+        //! one's address).  Only the null stream is always itself (the call costs 1.5 us of a list of
+        //! 1000 points' 80).  The lock is held from the sort to the record of `done` (several threads
+        //! may traverse at once); a copy of the traverser starts with none.
         struct QuerySorts
             {
             static constexpr size_t kMost = 4;
@@ -220,31 +222,32 @@ class LBVHTraverser : public Tunable<unsigned int>
 
         QuerySort& query_sort(stream_t stream)
             {
+            QuerySort& s = pick_sort(stream);
+            #ifdef HIP_API_PER_THREAD_DEFAULT_STREAM
+            const bool same = false;
+            #else
+            const bool same = !stream && !s.stream;
+            #endif
+            if (!same) NEIGHBOR_HIP_CHECK(hipStreamWaitEvent(stream, static_cast<hipEvent_t>(s.done.get()), 0));
+            s.stream = stream;
+            return s;
+            }
+        QuerySort& pick_sort(stream_t stream)
+            {
             for (QuerySort& s : m_sorts.all)
                 if (s.stream == stream) return s;
             for (QuerySort& s : m_sorts.all)
                 {
-                if (hipEventQuery(static_cast<hipEvent_t>(s.done.get())) == hipSuccess)
-                    {
-                    s.stream = stream;
-                    return s;
-                    }
+                if (hipEventQuery(static_cast<hipEvent_t>(s.done.get())) == hipSuccess) return s;
                 (void)hipGetLastError();    // not ready
                 }
-            if (m_sorts.all.size() < QuerySorts::kMost)
-                {
-                hipEvent_t e;
-                NEIGHBOR_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-                QuerySort s;
-                s.done = std::shared_ptr<void>(static_cast<void*>(e), [](void* p) { (void)hipEventDestroy(static_cast<hipEvent_t>(p)); });
-                s.stream = stream;
-                m_sorts.all.push_back(s);
-                return m_sorts.all.back();
-                }
-            QuerySort& s = m_sorts.all[m_sorts.oldest++ % QuerySorts::kMost];
-            NEIGHBOR_HIP_CHECK(hipStreamWaitEvent(stream, static_cast<hipEvent_t>(s.done.get()), 0));
-            s.stream = stream;
-            return s;
+            if (m_sorts.all.size() == QuerySorts::kMost) return m_sorts.all[m_sorts.oldest++ % QuerySorts::kMost];
+            hipEvent_t e;
+            NEIGHBOR_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            QuerySort s;
+            s.done = std::shared_ptr<void>(static_cast<void*>(e), [](void* p) { (void)hipEventDestroy(static_cast<hipEvent_t>(p)); });
+            m_sorts.all.push_back(s);
+            return m_sorts.all.back();
             }
 
         static bool capturing(stream_t stream)
