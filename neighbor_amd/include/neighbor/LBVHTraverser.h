@@ -220,6 +220,27 @@ class LBVHTraverser : public Tunable<unsigned int>
             QuerySorts& operator=(const QuerySorts&) { return *this; }
             } m_sorts;
 
+        //! Room for n queries in s: all of it or none.
+        static void grow(QuerySort& s, const unsigned int n, const size_t words, const bool both)
+            {
+            const auto room = [](shared_array<unsigned int>& kept, const size_t size) {
+                return size > kept.size() ? shared_array<unsigned int>(size, MemoryKind::Device) : shared_array<unsigned int>();
+            };
+            shared_array<unsigned int> keys[2], vals[2], work;
+            for (int i = 0; i < 2; ++i)
+                {
+                if (both) keys[i] = room(s.keys[i], n);
+                if (both || i == 0) vals[i] = room(s.vals[i], n);
+                }
+            work = room(s.work, words);
+            for (int i = 0; i < 2; ++i)
+                {
+                if (keys[i].size()) s.keys[i].swap(keys[i]);
+                if (vals[i].size()) s.vals[i].swap(vals[i]);
+                }
+            if (work.size()) s.work.swap(work);
+            }
+
         QuerySort& query_sort(stream_t stream)
             {
             QuerySort& s = pick_sort(stream);
@@ -264,19 +285,12 @@ class LBVHTraverser : public Tunable<unsigned int>
             const unsigned int bits = n <= (1u << 20) ? 16u : 24u;
             if (n <= gpu::radix::kernel::kRankSort)
                 {
-                if (n > s.vals[0].size()) shared_array<unsigned int>(n, MemoryKind::Device).swap(s.vals[0]);
+                grow(s, n, 0, false);
                 hipLaunchKernelGGL(gpu::kernel::query_order_ranked, dim3(div_up(n, 64)), dim3(gpu::radix::kernel::kRankBlock), 0, stream,
                                    spheres, n, m_lbvh_lo.get(), m_lbvh_hi.get(), bits, s.vals[0].get());
                 return s.vals[0].get();
                 }
-            const size_t words = gpu::radix::Workspace::words(n, bits);
-            if (n > s.keys[0].size())
-                for (int i = 0; i < 2; ++i)
-                    {
-                    shared_array<unsigned int>(n, MemoryKind::Device).swap(s.keys[i]);
-                    shared_array<unsigned int>(n, MemoryKind::Device).swap(s.vals[i]);
-                    }
-            if (words > s.work.size()) shared_array<unsigned int>(words, MemoryKind::Device).swap(s.work);
+            grow(s, n, gpu::radix::Workspace::words(n, bits), true);
             const gpu::radix::Workspace ws = gpu::radix::Workspace::carve(s.work.get(), n, bits);
             const size_t header = gpu::radix::Workspace::header_words(ws.passes);
             hipLaunchKernelGGL(gpu::radix::kernel::fill_zero, dim3(div_up(header, 256)), dim3(256), 0, stream, ws.hist, header);
@@ -298,10 +312,19 @@ class LBVHTraverser : public Tunable<unsigned int>
                 if (!order && query.size() > kSortQueries && !capturing(params.stream))
                     {
                     const std::lock_guard<std::mutex> guard(m_sorts.lock);
-                    QuerySort& sort = query_sort(params.stream);
-                    launch_front_in_order(params, query, out, images, sorted_queries(sort, query.spheres, query.size(), params.stream),
-                                          n_nodes, src);
-                    NEIGHBOR_HIP_CHECK(hipEventRecord(static_cast<hipEvent_t>(sort.done.get()), params.stream));
+                    QuerySort* sort = nullptr;
+                    const unsigned int* sorted = nullptr;
+                    try
+                        {
+                        sort = &query_sort(params.stream);
+                        sorted = sorted_queries(*sort, query.spheres, query.size(), params.stream);
+                        }
+                    catch (const hip_error& e)
+                        {
+                        if (e.code() != hipErrorOutOfMemory) throw;     // no room for the sort: served as they come
+                        }
+                    launch_front_in_order(params, query, out, images, sorted, n_nodes, src);
+                    if (sorted) NEIGHBOR_HIP_CHECK(hipEventRecord(static_cast<hipEvent_t>(sort->done.get()), params.stream));
                     return;
                     }
             launch_front_in_order(params, query, out, images, order, n_nodes, src);

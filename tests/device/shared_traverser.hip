@@ -3,8 +3,20 @@
 //
 // Usage: shared_traverser.bin MODE    prints OK and exits 0 on success
 //   threads  two host threads, each on its per-thread stream (one handle value for both)
+//   memory   the workspaces' allocations fail, one after the other
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+
+// The library's allocations, of which the one that counts the number down to zero fails.
+static std::atomic<int> g_fails_in{-1};
+template<class T>
+static hipError_t counted_malloc(T** p, const size_t size)
+    {
+    if (g_fails_in > 0 && --g_fails_in == 0) return hipErrorOutOfMemory;
+    return hipMalloc(p, size);
+    }
+#define hipMalloc(p, size) counted_malloc(p, size)
 #include "neighbor/neighbor.h"
 
 #include <cmath>
@@ -124,6 +136,26 @@ void threads()
     ta.join();
     tb.join();
     }
+
+void memory()
+    {
+    const System sys(30000, 4);
+    const std::shared_ptr<unsigned int> out = device<unsigned int>(sys.n);
+    const unsigned int sizes[] = {3000, 20000, 30000};
+    for (int fails_in = 1; fails_in <= 12; ++fails_in)
+        {
+        LBVHTraverser trav;
+        trav.setup(sys.lbvh);
+        g_fails_in = fails_in;
+        for (unsigned int k = 0; k < 9; ++k)
+            {
+            NEIGHBOR_HIP_CHECK(hipMemset(out.get(), 0xff, sys.n * sizeof(unsigned int)));
+            count(sys, trav, out.get(), sizes[k % 3u], 0);
+            check(sys, out.get(), sizes[k % 3u], "allocation " + std::to_string(fails_in) + " fails, call " + std::to_string(k));
+            }
+        g_fails_in = -1;
+        }
+    }
 } // end anonymous namespace
 
 int main(int argc, char** argv)
@@ -132,6 +164,7 @@ int main(int argc, char** argv)
     try
         {
         if (mode == "threads") threads();
+        else if (mode == "memory") memory();
         else return 2;
         }
     catch (const std::exception& e)

@@ -26,6 +26,39 @@ def test_threads_on_their_own_streams():
     run("threads")
 
 
+def test_no_memory_for_the_sort():
+    """Any of the workspaces' allocations may fail: the call is served unsorted, the next one right."""
+    run("memory")
+
+
+def test_unordered_under_capture():
+    """Unordered queries captured in a graph (not sorted there), replayed with eager calls between."""
+    import torch
+    import neighbor_amd as nb
+    n = 50000
+    rng = np.random.default_rng(23)
+    L = float(np.float32((n / 0.85) ** (1.0 / 3.0)))
+    pts = torch.from_numpy((rng.random((n, 3)) * L).astype(np.float32)).cuda()
+    lb = nb.LBVH()
+    lb.build(pts, [0, 0, 0], [L] * 3)
+    tr = nb.LBVHTraverser()
+    tr.setup(lb)
+    sets = [torch.cat([pts, torch.full((n, 1), r, device="cuda")], 1).contiguous() for r in (1.1, 1.4, 0.9)]
+    want = [tr.count(lb, s, order=lb.device_pointers()["primitive"]) for s in sets]
+    sph, out = sets[0].clone(), torch.zeros(n, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=stream):
+        tr.count(lb, sph, nneigh=out, stream=stream)
+    for s, w in zip(sets, want):
+        sph.copy_(s)
+        out.zero_()
+        graph.replay()
+        assert torch.equal(tr.count(lb, sph), w)
+        torch.cuda.synchronize()
+        assert torch.equal(out, w)
+
+
 def test_streams_across_the_sorts_limits():
     """Two streams and numbers of queries on both sides of the sorts' limits, in turn."""
     import torch
