@@ -220,6 +220,17 @@ class LBVHTraverser : public Tunable<unsigned int>
             QuerySorts& operator=(const QuerySorts&) { return *this; }
             } m_sorts;
 
+        //! Calls in its scope are not those that another thread's capture (global mode) forbids: they
+        //! allocate, free and ask events, on nothing that a capture uses.
+        struct BesideCaptures
+            {
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+            BesideCaptures() { NEIGHBOR_HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode)); }
+            ~BesideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+            BesideCaptures(const BesideCaptures&) = delete;
+            BesideCaptures& operator=(const BesideCaptures&) = delete;
+            };
+
         //! Room for n queries in s: all of it or none.
         static void grow(QuerySort& s, const unsigned int n, const size_t words, const bool both)
             {
@@ -312,6 +323,7 @@ class LBVHTraverser : public Tunable<unsigned int>
                 if (!order && query.size() > kSortQueries && !capturing(params.stream))
                     {
                     const std::lock_guard<std::mutex> guard(m_sorts.lock);
+                    const BesideCaptures beside;
                     QuerySort* sort = nullptr;
                     const unsigned int* sorted = nullptr;
                     try

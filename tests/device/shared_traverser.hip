@@ -4,6 +4,7 @@
 // Usage: shared_traverser.bin MODE    prints OK and exits 0 on success
 //   threads  two host threads, each on its per-thread stream (one handle value for both)
 //   memory   the workspaces' allocations fail, one after the other
+//   capture  beside another thread's capture in global mode
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -156,6 +157,53 @@ void memory()
         g_fails_in = -1;
         }
     }
+
+__global__ void mark(unsigned int* p)
+    {
+    *p = 7u;
+    }
+
+void capture()
+    {
+    const System sys(30000, 5);
+    LBVHTraverser trav;
+    trav.setup(sys.lbvh);
+    const std::shared_ptr<unsigned int> out = device<unsigned int>(sys.n), word = device<unsigned int>(1);
+    NEIGHBOR_HIP_CHECK(hipMemset(word.get(), 0, sizeof(unsigned int)));
+    hipStream_t captured, other;
+    NEIGHBOR_HIP_CHECK(hipStreamCreateWithFlags(&captured, hipStreamNonBlocking));
+    NEIGHBOR_HIP_CHECK(hipStreamCreateWithFlags(&other, hipStreamNonBlocking));
+    NEIGHBOR_HIP_CHECK(hipDeviceSynchronize());
+    NEIGHBOR_HIP_CHECK(hipStreamBeginCapture(captured, hipStreamCaptureModeGlobal));
+    std::string error;
+    try
+        {
+        // first uses, growth and a size that fits, beside the capture
+        const auto work = [&] {
+            for (const unsigned int nq : {3000u, 20000u, 30000u, 10000u}) count(sys, trav, out.get(), nq, other);
+        };
+        Thread<decltype(work)> t(work);
+        t.join();
+        }
+    catch (const std::exception& e) { error = e.what(); }
+    hipLaunchKernelGGL(mark, dim3(1), dim3(1), 0, captured, word.get());
+    hipGraph_t graph = nullptr;
+    const hipError_t ended = hipStreamEndCapture(captured, &graph);
+    if (!error.empty()) throw std::runtime_error("traversal beside a capture: " + error);
+    NEIGHBOR_HIP_CHECK(ended);
+    hipGraphExec_t exec;
+    NEIGHBOR_HIP_CHECK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
+    NEIGHBOR_HIP_CHECK(hipGraphLaunch(exec, captured));
+    NEIGHBOR_HIP_CHECK(hipDeviceSynchronize());
+    unsigned int got = 0;
+    NEIGHBOR_HIP_CHECK(hipMemcpy(&got, word.get(), sizeof(got), hipMemcpyDeviceToHost));
+    if (got != 7u) throw std::runtime_error("the captured kernel did not run");
+    check(sys, out.get(), 30000, "beside a capture");
+    NEIGHBOR_HIP_CHECK(hipGraphExecDestroy(exec));
+    NEIGHBOR_HIP_CHECK(hipGraphDestroy(graph));
+    NEIGHBOR_HIP_CHECK(hipStreamDestroy(captured));
+    NEIGHBOR_HIP_CHECK(hipStreamDestroy(other));
+    }
 } // end anonymous namespace
 
 int main(int argc, char** argv)
@@ -165,6 +213,7 @@ int main(int argc, char** argv)
         {
         if (mode == "threads") threads();
         else if (mode == "memory") memory();
+        else if (mode == "capture") capture();
         else return 2;
         }
     catch (const std::exception& e)

@@ -31,6 +31,11 @@ def test_no_memory_for_the_sort():
     run("memory")
 
 
+def test_beside_a_capture():
+    """Workspaces made and grown while another thread captures in global mode."""
+    run("capture")
+
+
 def test_unordered_under_capture():
     """Unordered queries captured in a graph (not sorted there), replayed with eager calls between."""
     import torch
