@@ -102,7 +102,7 @@ struct ExactSphereQueryOp
         Volume v;
         v.cd = make_double3(static_cast<double>(q.x) + t.x, static_cast<double>(q.y) + t.y, static_cast<double>(q.z) + t.z);
         v.c = make_float3(static_cast<float>(v.cd.x), static_cast<float>(v.cd.y), static_cast<float>(v.cd.z));
-        const double R = static_cast<double>(q.w);
+        const double R = fabs(static_cast<double>(q.w));     // only its square is defined
         v.R2 = R * R;
         const double cmax = fmax(fmax(fabs(v.cd.x), fabs(v.cd.y)), fabs(v.cd.z));
         const double Rpad = R * (1.0 + 0x1p-20) + cmax * 0x1p-21;

@@ -360,3 +360,21 @@ def test_exact_query_rope_records_by_size(nb, n):
     for variant in (nb.NB_VARIANT_QUANTIZED, nb.NB_VARIANT_FLOAT_ROPE, nb.NB_VARIANT_FLOAT_ROPE_EXACT):
         got = nb.LBVHTraverser(variant=variant).exact_count(lb, sph, d_pts, order=order)
         assert torch.equal(got, want)
+
+
+def test_exact_query_negative_radius(nb):
+    """Only the square of an exact query's radius counts, also at distances of exactly the radius and
+    where queries take a path each: lattice points have themselves and up to six neighbors."""
+    import torch
+    k = torch.arange(65, device="cuda", dtype=torch.float32)
+    pts = torch.stack(torch.meshgrid(k, k, k, indexing="ij"), -1).reshape(-1, 3).contiguous()
+    lb = nb.LBVH()
+    lb.build(pts, [0, 0, 0], [65.0] * 3)
+    want = 1 + sum((pts[:, a] > 0).int() + (pts[:, a] < 64).int() for a in range(3))
+    for radius in (1.0, -1.0):
+        sph = torch.cat([pts, torch.full((pts.shape[0], 1), radius, device="cuda")], 1).contiguous()
+        for variant in (nb.NB_VARIANT_FLOAT_ROPE_EXACT, nb.NB_VARIANT_QUANTIZED, nb.NB_VARIANT_WAVE):
+            tr = nb.LBVHTraverser(variant=variant)
+            for order in (None, lb.device_pointers()["primitive"]):
+                assert torch.equal(tr.exact_count(lb, sph, pts, order=order), want), (radius, variant)
+            assert torch.equal(tr.exact_count(lb, sph[:3000].contiguous(), pts), want[:3000])
