@@ -17,7 +17,7 @@
 #ifndef NEIGHBOR_KERNELS_FRONT_WALK_H_
 #define NEIGHBOR_KERNELS_FRONT_WALK_H_
 
-#include "LBVHTraverse.h"
+#include "WaveWalk.h"
 
 #include <new>
 #include <stdint.h>
@@ -256,14 +256,6 @@ __device__ __forceinline__ float4 anew(float4 v)
     {
     asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w));
     return v;
-    }
-
-//! Orders the wave's LDS accesses before and after it (one wave: no instruction).
-__device__ __forceinline__ void sync_lds()
-    {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
 
 __device__ __forceinline__ float lane_value(const float v, const unsigned int l)
@@ -548,7 +540,7 @@ __device__ __forceinline__ void write_hits(unsigned int* __restrict__ neigh, uns
                 }
             low = next;
             }
-        sync_lds();
+        wave::lds_order();
         for (uint32_t s = lane; s < total; s += 64u)
             {
             const unsigned int h = P.hit[s];
@@ -556,7 +548,7 @@ __device__ __forceinline__ void write_hits(unsigned int* __restrict__ neigh, uns
             neigh[to_pos] = P.prim[h & 63u];
             if (image) image[to_pos] = static_cast<unsigned char>(k);
             }
-        sync_lds();
+        wave::lds_order();
         }
     }
 
@@ -722,7 +714,7 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
             W.img[nimg - 1u - lane] = static_cast<uint8_t>(lane);
             if constexpr (SrcT::kFirst) W.first[nimg - 1u - lane] = 0u;
             }
-        sync_lds();
+        wave::lds_order();
         unsigned int cur = ~0u;                 // image of the open batch operands
         float half = 0.0f;                      // their bound of the leaf boxes' half diagonals
         float3 o = make_float3(0.0f, 0.0f, 0.0f);
@@ -766,7 +758,7 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
                 const unsigned long long im = wave::vote(reached && inner);
                 const unsigned long long lead = bm & (im ? (im & -im) - 1ull : ~0ull);    // buckets before the first inner node
                 const unsigned long long later = bm & ~lead;
-                sync_lds();
+                wave::lds_order();
                 if (wave::lane_in(lead))
                     W.list[ln + wave::count_below(lead)] = make_uint2(first, (end - first) | (k << 8) | (g << 16));
                 ln += static_cast<unsigned int>(__popcll(lead));
@@ -794,7 +786,7 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
                     W.img[to] = static_cast<uint8_t>(k);
                     if constexpr (SrcT::kFirst) W.first[to] = first;
                     }
-                sync_lds();
+                wave::lds_order();
                 continue;
                 }
 
@@ -873,10 +865,10 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
                 const double q2 = (static_cast<double>(x) * x + static_cast<double>(y) * y) + static_cast<double>(z) * z;
                 const double R = fabs(static_cast<double>(qq.w));
                 const double mid = kExact ? R * R : R * R + (R + 0.5 * half) * half;
-                sync_lds();
+                wave::lds_order();
                 W.local[lane] = takes_part ? make_float4(-2.0f * x, -2.0f * y, -2.0f * z, static_cast<float>(q2 - mid))
                                            : make_float4(0.0f, 0.0f, 0.0f, kNever);
-                sync_lds();
+                wave::lds_order();
                 operands();
             };
             operands();
@@ -978,7 +970,7 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
                     W.leaf[2u * kLeafStride + lane] = z;
                     W.leaf[3u * kLeafStride + lane] = w;
                     if constexpr (!kCount) P.prim[lane] = value;
-                    sync_lds();
+                    wave::lds_order();
                     uint32_t acc[4];
                     if constexpr (kExact)
                         {
@@ -1087,7 +1079,7 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
                         hits &= hits - 1ull;
                         }
                     }
-                sync_lds();
+                wave::lds_order();
                 }
             ln = 0u;
             }
@@ -1195,14 +1187,7 @@ __device__ __forceinline__ void lane_walk(const OutputOpT& out, const SrcT& src,
     typename OutputOpT::ThreadData result = out.setup(idx, q);
     unsigned int nimg = images.size() < 32u ? images.size() : 32u;
     if constexpr (kExact)
-        {
-        // no distance from a center that is not finite is within a finite radius, and none within or from
-        // a NaN: not walked, where box tests let such centers through everywhere
-        const float inf = __builtin_huge_valf();
-        const bool finite = fabsf(q.x) < inf && fabsf(q.y) < inf && fabsf(q.z) < inf;
-        const bool within = finite ? q.w == q.w : fabsf(q.w) == inf && q.x == q.x && q.y == q.y && q.z == q.z;
-        if (!within) nimg = 0u;
-        }
+        if (!wave::can_hit(q)) nimg = 0u;
     for (int pass = 0; pass < 2; ++pass)
         {
         for (unsigned int k = 0; k < nimg; ++k)
@@ -1247,6 +1232,24 @@ __device__ __forceinline__ void lane_walk(const OutputOpT& out, const SrcT& src,
         else if (!out.relocate(result)) break;
         }
     out.finalize(result);
+    }
+
+//! The walk of a wave's unusual queries, before that of the others (nothing of them is held in
+//! registers then).  lds: the wave's part.
+template<class SrcT, class OutputOpT, class QueryOpT, class TranslateOpT>
+__device__ __forceinline__ void walk_alone(const OutputOpT& out, const SrcT& src, const int root, const int stop, const BoundingBox& root_box,
+                                           const QueryOpT& query, const TranslateOpT& images, const bool mine, const unsigned int idx,
+                                           const float4& q, const unsigned int n_nodes, unsigned char* lds)
+    {
+    if constexpr (!SrcT::kFirst && std::is_same<QueryOpT, ExactSphereQueryOp>::value && wave::walks<OutputOpT>::value)
+        {
+        // a radius that reaches every point: 64 of a bucket's leaves at a time
+        static_assert(sizeof(wave::CompactWave) <= sizeof(FrontWave), "in the wave's part");
+        wave::walk(out, src.nodes, src.points, root_box, root, stop, query, images, src.transform, mine, idx, q, src.n_internal, n_nodes,
+                   *reinterpret_cast<wave::CompactWave*>(lds));
+        wave::lds_order();
+        }
+    else if (mine) lane_walk(out, src, root, stop, root_box, query, images, idx, q, n_nodes);
     }
 
 //! LDS of the front kernels: one part per wave, the second struct (not for counts) behind the first.
@@ -1350,18 +1353,12 @@ lbvh_traverse_front(const OutputOpT out,
     front::bind(src, root_box, bins);
     front::FrontWave& W = *reinterpret_cast<front::FrontWave*>(lds[wid]);
     front::FrontPairs& P = *reinterpret_cast<front::FrontPairs*>(lds[wid] + sizeof(front::FrontWave));
-    // unusual queries take a path of their own after the others' walk (their lanes are kept as a mask and
-    // they are read again: nothing of them is held in registers meanwhile)
-    const bool fronts = front::takes<SrcT, QueryOpT>(images, root_box);
-    const unsigned long long mine = wave::vote(valid && fronts && front::takes(q));
-    unsigned long long alone = wave::vote(valid) & ~mine;
-    if (mine && !front::walk<false>(out, src, root, root_box, query, images, wave::lane_in(mine), idx, q, n_nodes, W, P, nullptr))
-        alone |= mine;
-    if (wave::lane_in(alone))
-        {
-        const unsigned int i = order ? order[t] : t;
-        front::lane_walk(out, src, root, LBVHSentinel, root_box, query, images, i, query.setup(i), n_nodes);
-        }
+    const bool mine = valid && front::takes<SrcT, QueryOpT>(images, root_box) && front::takes(q);
+    if (__builtin_expect(wave::vote(valid && !mine) != 0ull, 0))
+        front::walk_alone(out, src, root, LBVHSentinel, root_box, query, images, valid && !mine, idx, q, n_nodes, lds[wid]);
+    if (wave::vote(mine) && front::walk<false>(out, src, root, root_box, query, images, mine, idx, q, n_nodes, W, P, nullptr)) return;
+    if (mine)
+        front::lane_walk(out, src, root, LBVHSentinel, root_box, query, images, idx, q, n_nodes);
     }
 
 //! lbvh_traverse_front with the four waves of a block for the same `per` (4, 16, 32 or 64) queries:
@@ -1395,16 +1392,12 @@ lbvh_traverse_team(const OutputOpT out,
     front::bind(src, root_box, bins);
     front::FrontWave& W = *reinterpret_cast<front::FrontWave*>(lds[wid]);
     front::FrontPairs& P = *reinterpret_cast<front::FrontPairs*>(lds[wid] + sizeof(front::FrontWave));
-    const bool fronts = front::takes<SrcT, QueryOpT>(images, root_box);
-    const unsigned long long mine = wave::vote(valid && fronts && front::takes(q));
-    unsigned long long alone = wave::vote(valid) & ~mine;
-    if (mine && !front::walk<true>(out, src, root, root_box, query, images, wave::lane_in(mine), idx, q, n_nodes, W, P, &team))
-        alone |= mine;
-    if (wid == 0u && wave::lane_in(alone))
-        {
-        const unsigned int i = order ? order[t] : t;
-        front::lane_walk(out, src, root, LBVHSentinel, root_box, query, images, i, query.setup(i), n_nodes);
-        }
+    const bool mine = valid && front::takes<SrcT, QueryOpT>(images, root_box) && front::takes(q);
+    if (__builtin_expect(wid == 0u && wave::vote(valid && !mine) != 0ull, 0))
+        front::walk_alone(out, src, root, LBVHSentinel, root_box, query, images, valid && !mine, idx, q, n_nodes, lds[wid]);
+    if (wave::vote(mine) && front::walk<true>(out, src, root, root_box, query, images, mine, idx, q, n_nodes, W, P, &team)) return;
+    if (mine && wid == 0u)
+        front::lane_walk(out, src, root, LBVHSentinel, root_box, query, images, idx, q, n_nodes);
     }
 
 } // end namespace kernel
