@@ -29,6 +29,7 @@
 #include "kernels/LBVHTraverse.h"
 
 #include <algorithm>
+#include <limits>
 #include <memory>
 #include <mutex>
 #include <stdexcept>
@@ -364,9 +365,70 @@ class LBVHTraverser : public Tunable<unsigned int>
             const unsigned int G = div_up(n, 256);
             const unsigned int x0 = G / 8u + (G % 8u ? 1u : 0u);
             const dim3 grid = tail ? dim3(8u * (x0 + (m_tail_split - 1u) * std::min(x0, tail))) : dim3(G);
-            hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_front<SourceT, OutputOpT, QueryOpT, TranslateOpT>), grid, dim3(256), 0,
-                               params.stream, out, src, m_lbvh_lo.get(), m_lbvh_hi.get(), m_bins.get(), m_root, query, images, order,
-                               n_nodes, tail, m_tail_split);
+            const auto fronts = [&](auto beside, const float limit) {
+                hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_front<decltype(beside)::value, SourceT, OutputOpT, QueryOpT, TranslateOpT>),
+                                   grid, dim3(256), 0, params.stream, out, src, m_lbvh_lo.get(), m_lbvh_hi.get(), m_bins.get(), m_root, query,
+                                   images, order, n_nodes, tail, m_tail_split, limit);
+            };
+            if constexpr (gpu::kernel::front::waves<SourceT, OutputOpT, QueryOpT>::value)
+                {
+                constexpr bool count = std::is_same<OutputOpT, CountNeighborsOp>::value;
+                const float limit = sparseLimit(!count, n, m_bucket, images.size());
+                if (limit > 0.0f)
+                    {
+                    launch_wave(params, query, out, images, order, n_nodes, src, limit);
+                    if constexpr (count) fronts(std::true_type(), limit);
+                    return;
+                    }
+                }
+            fronts(std::false_type(), 0.0f);
+            }
+
+        //! Exact counts and pair rows by one rope path per wave.
+        template<class OutputOpT, class TranslateOpT, class TransformOpT>
+        void launch_wave(const LaunchParameters& params, const ExactSphereQueryOp& query, const OutputOpT& out, const TranslateOpT& images,
+                         const unsigned int* order, const unsigned int n_nodes, const gpu::kernel::front::BucketSource<TransformOpT>& src,
+                         const float limit)
+            {
+            // the last wave that each SIMD of an XCD receives, in halves
+            const unsigned int tail = gpu::kernel::wave::places_rows<OutputOpT>::value ? 0u : m_tail_groups;
+            const unsigned int G = div_up(query.size(), 256);
+            const unsigned int x0 = G / 8u + (G % 8u ? 1u : 0u);
+            const dim3 grid = tail ? dim3(8u * (x0 + (m_tail_split - 1u) * std::min(x0, tail))) : dim3(G);
+            hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_wave<OutputOpT, TranslateOpT, TransformOpT>), grid, dim3(256), 0, params.stream,
+                               out, src, m_lbvh_lo.get(), m_lbvh_hi.get(), m_root, query, images, order, n_nodes, tail, m_tail_split, limit);
+            }
+
+        //! Exact queries over bucket records: the walk by node fronts serves those with more leaves within
+        //! their radius than this, one rope path per wave the others (0: fronts only; infinite, rows: never).
+        /*!
+         * Fronts take a third of the dependent steps with half the waves on the chip: they win where one
+         * wave's chain is long (dense neighbors, images, small buckets), lose where the launch is many
+         * rounds of short walks.  Measured with uniform points at density 0.85 and radii 1.5, 2 and 2.8
+         * (13, 29 and 79 neighbors), one rope path per wave against fronts in us:
+         *  - Counts, no images, 64 leaves per bucket: 300,000 points 111/114, 135/123, 184/159; 10^6
+         *    249/306, 302/325, 423/345; 4 10^6 862/1185, 1074/1230, 1542/1563.  16 leaves: 10^6 333/306,
+         *    394/366, 514/427.  27 images, 64 leaves: 10^6 308/327, 371/351, 483/374; 2 10^6 532/639,
+         *    630/656, 874/814.  The radius decides, and only the device knows it: both kernels are launched
+         *    and one leaves at once (5 to 9 us), where the limit is not below 8 (about the fewest leaves
+         *    per radius in use) and, with images, above 2^20 queries.
+         *  - Rows depend less on it.  No images, 64 leaves: 200,000 108/120, 127/126, 173/159; 300,000
+         *    128/159, 151/177, 217/251; 10^6 289/408, 350/458, 506/557; 32 leaves: 300,000 138/148,
+         *    164/164, 237/259, 10^6 306/384, 370/442, 531/550; 16 leaves: 10^6 366/386, 452/484, 666/634.
+         *    27 images, 64 leaves: 700,000 295/311, 343/349, 442/418, 10^6 374/433, 453/487, 611/601; 32
+         *    leaves: 10^6 398/403, 469/472, 641/586, 2 10^6 683/773, 842/849, 1268/1380.
+         * Left: rows with images of sparse queries (5 neighbors, 10^6, 64 leaves: 314/403), and rows of
+         * 300,000 dense ones with images (64 leaves 254/278).
+         */
+        static float sparseLimit(const bool rows, const unsigned int n, const unsigned int bucket, const unsigned int images)
+            {
+            const float size = static_cast<float>(n) * 0x1p-20f, leaves = static_cast<float>(bucket);
+            constexpr float never = std::numeric_limits<float>::infinity();
+            if (n <= kFrontsOnly) return 0.0f;
+            if (rows) return bucket >= 24u && (images == 1u || size * leaves > 48.0f) ? never : 0.0f;
+            if (images > 1u && n <= 4u * kFrontsOnly) return 0.0f;
+            const float limit = (images == 1u ? 0.6f : 0.3f) * leaves * std::min(leaves * 0x1p-5f, 1.0f) * size;
+            return limit < 8.0f ? 0.0f : limit;
             }
 
         //! Rope and quantized records by node fronts; false: not this query op, or too many exact queries.
@@ -474,6 +536,7 @@ class LBVHTraverser : public Tunable<unsigned int>
         //! for 16 and for 4: 1000 points 35 and 47 us, 29 and 38; 4000 points 56 and 72, 45 and 56;
         //! 8000 points 48 and 65, 62 and 77.
         static constexpr unsigned int kTeamQueries = 1u << 16;
+        static constexpr unsigned int kFrontsOnly = 1u << 18;
         //! Tail split (wave::tail_block): per XCD, the last groups of 256 queries run as m_tail_split
         //! blocks each, so that the waves that start last are shorter.  Up to kAllSplit queries, which
         //! leave wave slots free, all groups do (64 per XCD), up to kHalfSplit 32 of each XCD, above it

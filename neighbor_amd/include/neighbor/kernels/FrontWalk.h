@@ -563,6 +563,49 @@ union Slot
     __device__ ~Slot() {}
     };
 
+//! Boxes around each quad of lanes' queries, and their largest radius (in all of its lanes).
+struct Quad
+    {
+    float3 lo, hi;
+    float r;
+    };
+__device__ __forceinline__ Quad quad_of(const bool act, const float4& q)
+    {
+    return Quad{make_float3(quad_min(act ? q.x : kNever), quad_min(act ? q.y : kNever), quad_min(act ? q.z : kNever)),
+                make_float3(-quad_min(act ? -q.x : kNever), -quad_min(act ? -q.y : kNever), -quad_min(act ? -q.z : kNever)),
+                -quad_min(act ? -fabsf(q.w) : 0.0f)};
+    }
+__device__ __forceinline__ float volume(const BoundingBox& b)
+    {
+    return fmaxf(b.hi.x - b.lo.x, 0.0f) * fmaxf(b.hi.y - b.lo.y, 0.0f) * fmaxf(b.hi.z - b.lo.z, 0.0f);
+    }
+//! Side of the cube that holds one of the tree's leaves on average.
+__device__ __forceinline__ float mean_cell(const BoundingBox& root_box, const unsigned int n_nodes)
+    {
+    const float leaves = 0.5f * static_cast<float>(n_nodes + 1u);
+    return exp2f(log2f(volume(root_box) / leaves) * (1.0f / 3.0f));
+    }
+//! Lanes of the groups or quads whose box is mostly empty.
+__device__ __forceinline__ unsigned long long mostly_empty(const float3& lo, const float3& hi, const float radius, const float cell)
+    {
+    return wave::vote(fmaxf(fmaxf(hi.x - lo.x, hi.y - lo.y), hi.z - lo.z) > fmaxf(kSpreadRadii * radius, kSpreadCells * cell));
+    }
+//! Queries all over the tree (qwide: mostly_empty of the quads): a front, or one path for the wave,
+//! would walk the union of their paths.
+__device__ __forceinline__ bool scattered(const unsigned long long act, const unsigned long long qwide, const unsigned int n_nodes)
+    {
+    return n_nodes > kSmallTree && 8u * static_cast<unsigned int>(__popcll(qwide)) > kScattered * static_cast<unsigned int>(__popcll(act));
+    }
+
+//! True when few leaves are expected within the radius of the launch's first query (fewer than limit).
+template<class QueryOpT>
+__device__ __forceinline__ bool sparse(const QueryOpT& query, const unsigned int* __restrict__ order, const BoundingBox& root_box,
+                                       const unsigned int n_nodes, const float limit)
+    {
+    const float R = fabsf(query.spheres[order ? order[0] : 0u].w);
+    return 4.18879f * R * R * R * (0.5f * static_cast<float>(n_nodes + 1u)) < limit * volume(root_box);
+    }
+
 //! The walk over the subtree of `root` (n_nodes nodes) for one query per lane, by one wave or, TEAM,
 //! by the four waves of a block for the same queries; false: not walked (queries too scattered).
 /*!
@@ -646,9 +689,9 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
         float rmax;
         float3 center;                          // of the wave's queries: its origin before the image vector
         {
-        const float3 qlo = make_float3(quad_min(act ? q.x : kNever), quad_min(act ? q.y : kNever), quad_min(act ? q.z : kNever));
-        const float3 qhi = make_float3(-quad_min(act ? -q.x : kNever), -quad_min(act ? -q.y : kNever), -quad_min(act ? -q.z : kNever));
-        const float qrr = -quad_min(act ? -r : 0.0f);
+        const Quad quad = quad_of(act, q);
+        const float3 qlo = quad.lo, qhi = quad.hi;
+        const float qrr = quad.r;
         const float3 glo = make_float3(over_quads_min(qlo.x), over_quads_min(qlo.y), over_quads_min(qlo.z));
         const float3 ghi = make_float3(-over_quads_min(-qhi.x), -over_quads_min(-qhi.y), -over_quads_min(-qhi.z));
         const float grr = -over_quads_min(-qrr);
@@ -672,25 +715,18 @@ __device__ __forceinline__ bool walk(const OutputOpT& out, const SrcT& src, cons
             W.lo[lane >> 4] = make_float4(glo.x, glo.y, glo.z, padded(grr));
             W.hi[lane >> 4] = make_float4(ghi.x, ghi.y, ghi.z, 0.0f);
             }
-        // side of the cube that holds one of the tree's leaves on average
-        const float leaves = 0.5f * static_cast<float>(n_nodes + 1u);
-        const float cell = exp2f(log2f(fmaxf(root_box.hi.x - root_box.lo.x, 0.0f) * fmaxf(root_box.hi.y - root_box.lo.y, 0.0f)
-                                       * fmaxf(root_box.hi.z - root_box.lo.z, 0.0f) / leaves) * (1.0f / 3.0f));
-        const auto wider = [](const float3& a, const float3& b, const float side) {
-            return wave::vote(fmaxf(fmaxf(b.x - a.x, b.y - a.y), b.z - a.z) > side);
-        };
-        const unsigned long long wide = wider(glo, ghi, fmaxf(kSpreadRadii * grr, kSpreadCells * cell)),
-                                 qwide = wider(qlo, qhi, fmaxf(kSpreadRadii * qrr, kSpreadCells * cell));
+        const float cell = mean_cell(root_box, n_nodes);
+        const unsigned long long wide = mostly_empty(glo, ghi, grr, cell), qwide = mostly_empty(qlo, qhi, qrr, cell);
         #pragma unroll
         for (unsigned int g = 0; g < 4; ++g)
             {
             if ((actm >> (16u * g)) & 0xffffull) active |= 1u << g;
             if ((wide >> (16u * g)) & 1ull) spread |= 1u << g;
             }
-        // queries all over the tree: a front would walk the union of their paths (the few queries of
-        // a team are still walked faster by its four waves than one per lane: 4000 spheres of
-        // radius 5.9 in a tree of 396,000 points, 16 per team, 123 us against 185)
-        if (pass == 0 && n_nodes > kSmallTree && (!TEAM || __popcll(actm) > 16) && 8u * static_cast<unsigned int>(__popcll(qwide)) > kScattered * static_cast<unsigned int>(__popcll(actm))) return false;
+        // the few queries of a team are walked faster by its four waves than one per lane also where
+        // they are scattered: 4000 spheres of radius 5.9 in a tree of 396,000 points, 16 per team, 123
+        // us against 185
+        if (pass == 0 && (!TEAM || __popcll(actm) > 16) && scattered(actm, qwide, n_nodes)) return false;
         if constexpr (!kCount && !kRows)
             if (pass == 0 && valid) new (&slot.data) typename OutputOpT::ThreadData(out.setup(idx, q));
         if (spread && qwide)
@@ -1234,6 +1270,12 @@ __device__ __forceinline__ void lane_walk(const OutputOpT& out, const SrcT& src,
     out.finalize(result);
     }
 
+//! Launches that the walk by one rope path per wave can serve, too.
+template<class SrcT, class OutputOpT, class QueryOpT>
+struct waves
+    : std::integral_constant<bool, !SrcT::kFirst && std::is_same<QueryOpT, ExactSphereQueryOp>::value && wave::walks<OutputOpT>::value>
+    {};
+
 //! The walk of a wave's unusual queries, before that of the others (nothing of them is held in
 //! registers then).  lds: the wave's part.
 template<class SrcT, class OutputOpT, class QueryOpT, class TranslateOpT>
@@ -1241,7 +1283,7 @@ __device__ __forceinline__ void walk_alone(const OutputOpT& out, const SrcT& src
                                            const QueryOpT& query, const TranslateOpT& images, const bool mine, const unsigned int idx,
                                            const float4& q, const unsigned int n_nodes, unsigned char* lds)
     {
-    if constexpr (!SrcT::kFirst && std::is_same<QueryOpT, ExactSphereQueryOp>::value && wave::walks<OutputOpT>::value)
+    if constexpr (waves<SrcT, OutputOpT, QueryOpT>::value)
         {
         // a radius that reaches every point: 64 of a bucket's leaves at a time
         static_assert(sizeof(wave::CompactWave) <= sizeof(FrontWave), "in the wave's part");
@@ -1321,8 +1363,9 @@ __global__ void __launch_bounds__(radix::kernel::kRankBlock) query_order_ranked(
     }
 
 //! Traversal by node fronts, one wave per 64 consecutive queries of the traversal order.  Blocks
-//! map to queries by wave::tail_block.
-template<class SrcT, class OutputOpT, class QueryOpT, class TranslateOpT>
+//! map to queries by wave::tail_block.  BESIDE: launched beside lbvh_traverse_wave, which serves the
+//! queries when few leaves (fewer than limit) are within their radius.
+template<bool BESIDE, class SrcT, class OutputOpT, class QueryOpT, class TranslateOpT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
 lbvh_traverse_front(const OutputOpT out,
                     SrcT src,
@@ -1335,7 +1378,8 @@ lbvh_traverse_front(const OutputOpT out,
                     const unsigned int* __restrict__ order,
                     const unsigned int n_nodes,
                     const unsigned int tail_groups,
-                    const unsigned int tail_split)
+                    const unsigned int tail_split,
+                    const float limit)
     {
     typedef front::FrontLds<OutputOpT> Lds;
     __shared__ alignas(16) unsigned char lds[4][Lds::kPart];
@@ -1345,20 +1389,66 @@ lbvh_traverse_front(const OutputOpT out,
     const unsigned int lane = threadIdx.x & 63u;
     const unsigned int wid = static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)));
     const unsigned int t = span.first + wid * span.per_wave + lane;
-    const bool valid = lane < span.per_wave && t < n;
+    bool valid = lane < span.per_wave && t < n;
     const unsigned int idx = valid ? (order ? order[t] : t) : 0u;
+    const BoundingBox root_box(*root_lo, *root_hi);
+    if constexpr (BESIDE)
+        if (front::sparse(query, order, root_box, n_nodes, limit)) return;
     wave::place_rows(out, t, idx, valid);
     const float4 q = valid ? query.setup(idx) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    const BoundingBox root_box(*root_lo, *root_hi);
     front::bind(src, root_box, bins);
     front::FrontWave& W = *reinterpret_cast<front::FrontWave*>(lds[wid]);
     front::FrontPairs& P = *reinterpret_cast<front::FrontPairs*>(lds[wid] + sizeof(front::FrontWave));
-    const bool mine = valid && front::takes<SrcT, QueryOpT>(images, root_box) && front::takes(q);
-    if (__builtin_expect(wave::vote(valid && !mine) != 0ull, 0))
-        front::walk_alone(out, src, root, LBVHSentinel, root_box, query, images, valid && !mine, idx, q, n_nodes, lds[wid]);
-    if (wave::vote(mine) && front::walk<false>(out, src, root, root_box, query, images, mine, idx, q, n_nodes, W, P, nullptr)) return;
-    if (mine)
+    const bool odd = valid && !(front::takes(q) && front::takes<SrcT, QueryOpT>(images, root_box));
+    if (__builtin_expect(wave::vote(odd) != 0ull, 0))
+        {
+        front::walk_alone(out, src, root, LBVHSentinel, root_box, query, images, odd, idx, q, n_nodes, lds[wid]);
+        valid = valid && !odd;
+        }
+    if (front::walk<false>(out, src, root, root_box, query, images, valid, idx, q, n_nodes, W, P, nullptr)) return;
+    if (valid)
         front::lane_walk(out, src, root, LBVHSentinel, root_box, query, images, idx, q, n_nodes);
+    }
+
+//! Exact counts and pair rows by one rope path per wave for 64 consecutive queries (wave::walk).
+//! Blocks map to queries by wave::tail_block.  A finite limit: launched beside lbvh_traverse_front,
+//! which serves the queries unless fewer leaves than limit are within their radius.
+template<class OutputOpT, class TranslateOpT, class TransformOpT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8)))
+lbvh_traverse_wave(const OutputOpT out,
+                   const front::BucketSource<TransformOpT> src,
+                   const float3* __restrict__ root_lo,
+                   const float3* __restrict__ root_hi,
+                   const int root,
+                   const ExactSphereQueryOp query,
+                   const TranslateOpT images,
+                   const unsigned int* __restrict__ order,
+                   const unsigned int n_nodes,
+                   const unsigned int tail_groups,
+                   const unsigned int tail_split,
+                   const float limit)
+    {
+    __shared__ wave::CompactWave lds[4];
+    const unsigned int n = query.size();
+    const wave::BlockSpan span = wave::tail_block(blockIdx.x, (n + 255u) / 256u, tail_groups, tail_split);
+    if (!span.live) return;
+    const unsigned int lane = threadIdx.x & 63u;
+    const unsigned int t = span.first + (threadIdx.x >> 6) * span.per_wave + lane;
+    const bool valid = lane < span.per_wave && t < n;
+    const unsigned int idx = valid ? (order ? order[t] : t) : 0u;
+    const BoundingBox root_box(*root_lo, *root_hi);
+    if (limit < __builtin_huge_valf() && !front::sparse(query, order, root_box, n_nodes, limit)) return;
+    wave::place_rows(out, t, idx, valid);
+    const float4 q = valid ? query.setup(idx) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const front::Quad quad = front::quad_of(valid, q);
+    const unsigned long long qwide = front::mostly_empty(quad.lo, quad.hi, quad.r, front::mean_cell(root_box, n_nodes));
+    if (__builtin_expect(front::scattered(wave::vote(valid), qwide, n_nodes), 0))
+        {
+        if (valid) front::lane_walk(out, src, root, LBVHSentinel, root_box, query, images, idx, q, n_nodes);
+        return;
+        }
+    wave::walk(out, src.nodes, src.points, root_box, root, LBVHSentinel, query, images, src.transform, valid, idx, q, src.n_internal,
+               n_nodes, lds[threadIdx.x >> 6]);
     }
 
 //! lbvh_traverse_front with the four waves of a block for the same `per` (4, 16, 32 or 64) queries:
@@ -1385,18 +1475,21 @@ lbvh_traverse_team(const OutputOpT out,
     const unsigned int lane = threadIdx.x & 63u;
     const unsigned int wid = static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)));
     const unsigned int t = per * wave::xcd_block(blockIdx.x, gridDim.x) + lane;
-    const bool valid = lane < per && t < n;
+    bool valid = lane < per && t < n;
     const unsigned int idx = valid ? (order ? order[t] : t) : 0u;
     const float4 q = valid ? query.setup(idx) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     const BoundingBox root_box(*root_lo, *root_hi);
     front::bind(src, root_box, bins);
     front::FrontWave& W = *reinterpret_cast<front::FrontWave*>(lds[wid]);
     front::FrontPairs& P = *reinterpret_cast<front::FrontPairs*>(lds[wid] + sizeof(front::FrontWave));
-    const bool mine = valid && front::takes<SrcT, QueryOpT>(images, root_box) && front::takes(q);
-    if (__builtin_expect(wid == 0u && wave::vote(valid && !mine) != 0ull, 0))
-        front::walk_alone(out, src, root, LBVHSentinel, root_box, query, images, valid && !mine, idx, q, n_nodes, lds[wid]);
-    if (wave::vote(mine) && front::walk<true>(out, src, root, root_box, query, images, mine, idx, q, n_nodes, W, P, &team)) return;
-    if (mine && wid == 0u)
+    const bool odd = valid && !(front::takes(q) && front::takes<SrcT, QueryOpT>(images, root_box));
+    if (__builtin_expect(wave::vote(odd) != 0ull, 0))
+        {
+        if (wid == 0u) front::walk_alone(out, src, root, LBVHSentinel, root_box, query, images, odd, idx, q, n_nodes, lds[wid]);
+        valid = valid && !odd;
+        }
+    if (front::walk<true>(out, src, root, root_box, query, images, valid, idx, q, n_nodes, W, P, &team)) return;
+    if (valid && wid == 0u)
         front::lane_walk(out, src, root, LBVHSentinel, root_box, query, images, idx, q, n_nodes);
     }
 

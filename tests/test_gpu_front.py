@@ -378,3 +378,66 @@ def test_exact_query_negative_radius(nb):
             for order in (None, lb.device_pointers()["primitive"]):
                 assert torch.equal(tr.exact_count(lb, sph, pts, order=order), want), (radius, variant)
             assert torch.equal(tr.exact_count(lb, sph[:3000].contiguous(), pts), want[:3000])
+
+
+# around the launches that one rope path per wave serves: from 2^18 queries, by rows or counts, leaves
+# per bucket, images and (counts) radius
+@pytest.mark.parametrize("n,bucket,images,radius", [
+    (262144, 64, False, 1.0), (262145, 64, False, 1.0), (262145, 24, False, 1.4), (262145, 23, False, 1.4),
+    (600001, 64, False, 1.0), (600001, 64, False, 1.9), (800003, 64, True, 1.0), (1048577, 32, True, 0.9),
+    (1048577, 64, True, 0.8)])
+@pytest.mark.parametrize("given", ["tree", "random", None])
+def test_many_exact_queries(nb, n, bucket, images, radius, given):
+    """Counts and rows, as given, placed and all moved, equal those of a path per query."""
+    import torch
+    from neighbor_amd.api import exact_rows, exclusive_scan
+    from neighbor_amd.learned import exact_rows_placed
+    from neighbor_amd.workloads import images27
+    if given != "tree" and n > 600001:
+        pytest.skip("the largest in the tree's order only")
+    rng = np.random.default_rng(n + bucket)
+    pts, L = points_of(n, rng, "uniform")
+    d_pts = torch.from_numpy(pts).cuda()
+    sph = torch.cat([d_pts, torch.full((n, 1), radius, device="cuda")], 1).contiguous()
+    sph[12345, 0] = float("nan")
+    sph[54321, 3] = -radius
+    img = torch.from_numpy(images27(L, dtype=np.float64)).cuda() if images else None
+    lb = nb.LBVH()
+    lb.build(d_pts, [0, 0, 0], [L] * 3)
+    prim = lb.arrays()["primitive"].long()
+    tree = lb.device_pointers()["primitive"]
+    order = {"tree": tree, "random": torch.from_numpy(rng.permutation(n).astype(np.int32)).cuda(), None: None}[given]
+
+    def rows(variant, order):
+        tr = nb.LBVHTraverser(variant=variant)
+        tr.set_bucket_size(bucket)
+        tr.setup(lb)
+        counts = tr.exact_count(lb, sph, d_pts, images=img, order=order)
+        start = exclusive_scan(counts, perm=tree)
+        neigh = torch.full((int(counts.sum()),), -1, dtype=torch.int32, device="cuda")
+        image = torch.full((neigh.numel(),), 77, dtype=torch.uint8, device="cuda")
+        exact_rows(tr, lb, sph, d_pts, start, counts, neigh, image, images=img, order=order)
+        return tr, counts, start, neigh, image
+
+    _, counts, start, neigh, image = rows(nb.NB_VARIANT_FLOAT_ROPE_EXACT, tree)
+    tr, *got = rows(nb.NB_VARIANT_WAVE, order)
+    for g, w in zip(got, (counts, start, neigh, image)):
+        assert torch.equal(g, w)
+    if given != "tree":
+        return
+    for moved in (False, True):
+        cap = counts // 2 if moved else counts.clone()
+        sums = torch.zeros(((n + 255) // 256 * 256,), dtype=torch.int64, device="cuda")
+        sums[:n] = cap[prim].long()
+        base = torch.zeros((n + 255) // 256 + 1, dtype=torch.int64, device="cuda")
+        base[1:] = sums.view(-1, 256).sum(1).cumsum(0)
+        used = int(base[-1])
+        spill = torch.tensor([used, 0], dtype=torch.int64, device="cuda")
+        to = torch.full((used + neigh.numel(),), -1, dtype=torch.int32, device="cuda")
+        to_image = torch.full((to.numel(),), 77, dtype=torch.uint8, device="cuda")
+        at, nn = torch.zeros(n + 1, dtype=torch.int64, device="cuda"), torch.zeros_like(counts)
+        exact_rows_placed(tr, lb, sph, d_pts, base, at, cap, to, to_image, nn, spill=spill, images=img)
+        assert torch.equal(nn, counts)
+        rest = torch.arange(neigh.numel(), device="cuda") - torch.repeat_interleave(start[:n][prim], counts[prim].long())
+        where = torch.repeat_interleave(at[:n][prim], counts[prim].long()) + rest
+        assert torch.equal(to[where], neigh) and torch.equal(to_image[where], image)
