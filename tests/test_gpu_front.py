@@ -441,3 +441,54 @@ def test_many_exact_queries(nb, n, bucket, images, radius, given):
         rest = torch.arange(neigh.numel(), device="cuda") - torch.repeat_interleave(start[:n][prim], counts[prim].long())
         where = torch.repeat_interleave(at[:n][prim], counts[prim].long()) + rest
         assert torch.equal(to[where], neigh) and torch.equal(to_image[where], image)
+
+
+@pytest.mark.parametrize("nq", [20000, 32768, 40001])
+@pytest.mark.parametrize("images", [False, True])
+def test_scattered_teams(nb, orc, nq, images):
+    """Queries in random order served by teams of 32 and 64, in a tree in which such queries take a path
+    each: lists and exact rows in the walks' order, and rows that all move."""
+    import torch
+    from neighbor_amd.api import exact_rows, exclusive_scan
+    from neighbor_amd.workloads import images27
+    rng = np.random.default_rng(nq)
+    n = 40001
+    pts, L = points_of(n, rng, "uniform")
+    sph = np.concatenate([rng.random((nq, 3)) * L, rng.uniform(0.5, 1.4, (nq, 1))], 1).astype(np.float32)
+    sph[77, 1] = np.nan
+    imgs = images27(L)
+    d_pts, d_sph = torch.from_numpy(pts).cuda(), torch.from_numpy(sph).cuda()
+    lb = nb.LBVH()
+    lb.build(d_pts, [0, 0, 0], [L] * 3)
+    order = torch.from_numpy(rng.permutation(nq).astype(np.int32)).cuda()
+    ref = orc.traverse(n, orc.compress(orc.build(pts, [0, 0, 0], [L] * 3)), sph, imgs if images else None, triplets=True)
+    want = ref["counts"].astype(np.int64)
+    starts = np.concatenate([[0], np.cumsum(want)])
+    f32 = torch.from_numpy(imgs).cuda() if images else None
+    f64 = torch.from_numpy(imgs.astype(np.float64)).cuda() if images else None
+    for variant in (nb.NB_VARIANT_QUANTIZED, nb.NB_VARIANT_WAVE_QUANTIZED):
+        tr = nb.LBVHTraverser(variant=variant)
+        assert np.array_equal(host(tr.count(lb, d_sph, images=f32, order=order)).astype(np.int64), want)
+        neigh, image = tr.pairs(lb, d_sph, torch.from_numpy(starts).cuda(), images=f32, order=order)
+        assert np.array_equal(host(neigh).astype(np.int64), ref["prim"].astype(np.int64))
+        assert np.array_equal(host(image), ref["image"])
+    rows = []
+    for variant in (nb.NB_VARIANT_FLOAT_ROPE_EXACT, nb.NB_VARIANT_WAVE):
+        tr = nb.LBVHTraverser(variant=variant)
+        counts = tr.exact_count(lb, d_sph, d_pts, images=f64, order=order)
+        start = exclusive_scan(counts)
+        total = int(start[-1])
+        neigh = torch.full((total,), -1, dtype=torch.int32, device="cuda")
+        exact_rows(tr, lb, d_sph, d_pts, start, counts, neigh, images=f64, order=order)
+        # no room at first: every row that has pairs moves
+        moved, cap = start.clone(), torch.zeros_like(counts)
+        to = torch.full((2 * total,), -1, dtype=torch.int32, device="cuda")
+        spill = torch.tensor([total, 0], dtype=torch.int64, device="cuda")
+        got = exact_rows(tr, lb, d_sph, d_pts, moved, cap, to, images=f64, order=order, spill=spill)
+        assert torch.equal(got, counts) and int(spill[0]) == 2 * total
+        at = torch.arange(total, device="cuda") + torch.repeat_interleave(moved[:nq] - start[:nq], counts.long())
+        assert torch.equal(to[at], neigh)
+        rows.append((host(counts), host(neigh)))
+    assert np.array_equal(rows[0][0], rows[1][0]) and np.array_equal(rows[0][1], rows[1][1])
+    ref = orc.exact_bruteforce(pts, sph[:2000], imgs.astype(np.float64) if images else np.zeros((1, 3)), pairs=False)
+    assert np.array_equal(rows[0][0][:2000].view(np.uint32), ref["counts"])
