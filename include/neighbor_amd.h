@@ -319,7 +319,8 @@ int nb_batch_build(nb_batch* batch, const float* points, uint32_t N, const uint3
                    const float* box_hi, uint32_t nbox, void* stream);
 /* Tunables: block (hierarchy kernel, multiple of 32 in [32, 1024]), bucket (leaves per bucket,
  * 1..64), variant (NB_BATCH_*), grid (blocks of the traversal, 0 = one wave per 64 queries of a
- * box).  Bucket changes take effect at nb_batch_setup. */
+ * box).  Bucket changes take effect at nb_batch_setup.  nb_batch_get_params returns what was set
+ * (or chosen by nb_batch_tune), whatever is built. */
 int nb_batch_set_params(nb_batch* batch, uint32_t block, uint32_t bucket, int variant, uint32_t grid);
 int nb_batch_get_params(const nb_batch* batch, uint32_t* block, uint32_t* bucket, int* variant, uint32_t* grid);
 /* Bucket records of the built forest (after every build). */

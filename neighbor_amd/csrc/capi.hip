@@ -742,7 +742,7 @@ int nb_batch_get_params(const nb_batch* b, uint32_t* block, uint32_t* bucket, in
         if (block) *block = b->batch.getBlock();
         if (bucket) *bucket = b->batch.getBucket();
         if (variant) *variant = b->variant == neighbor::BatchVariant::Lane ? NB_BATCH_LANE : NB_BATCH_WAVE;
-        if (grid) *grid = b->batch.gridSize();
+        if (grid) *grid = b->batch.getGrid();
     });
     }
 

@@ -199,6 +199,7 @@ class LBVHBatch
         unsigned int getBucket() const { return m_bucket; }
         //! Blocks of the traversal (0: one wave per work item).
         void setGrid(unsigned int g) { m_grid = g; }
+        unsigned int getGrid() const { return m_grid; }
 
         unsigned int getN() const { return m_N; }
         unsigned int getNBoxes() const { return m_nbox; }
