@@ -440,7 +440,7 @@ class LBVHTraverser : public Tunable<unsigned int>
             constexpr bool reference = std::is_same<QueryOpT, SphereQueryOp>::value;
             if constexpr (exact || reference)
                 {
-                if (exact && query.size() > kRopeFronts) return false;
+                if (exact && m_variant != TraversalVariant::Quantized && query.size() > kRopeFronts) return false;
                 if (m_variant == TraversalVariant::Quantized)
                     launch_front(params, query, out, images, order, lbvh.getNNodes(),
                                  gpu::kernel::front::QuantizedSource{m_data.get(), float3(), float3(), float3(), lbvh.getNInternal()});
@@ -524,10 +524,14 @@ class LBVHTraverser : public Tunable<unsigned int>
         //! images: 256 queries 44 us and 44, 512 71 and 54, 1000 89 and 44; without images 14 and 24,
         //! 21 and 30, 34 and 33; 10^6 (one rope path per lane) 8.2 ms and 0.7.
         static constexpr unsigned int kSortQueries = 256;
-        //! Exact queries over rope records up to which they walk by fronts.  These records are the choice
-        //! for few neighbors per query, where a walk is one short path down from the root: by fronts and
-        //! by a path per lane, 99,000 queries of 4 neighbors 75 and 100 us, 396,000 157 and 167, 990,000
-        //! 322 and 267 (1000 to 10,000 large ones in the same trees 50 to 151 and 229 to 395).
+        //! Exact queries over float rope records up to which they walk by fronts (quantized ones: any
+        //! number).  These records are the choice for few neighbors per query, where a walk is one short
+        //! path down from the root.  Exact counts by a path per lane and by fronts, uniform points: 262,144
+        //! queries of 2.5 neighbors 100/114 us, of 5 126/118; 330,000 106/133, 124/142 (3.6), 150/146 (5),
+        //! 263/148 (13); 524,288 167/185, 213/194, 269/199, 498/208; 990,000 275/339, 340/351, 424/359,
+        //! 836/371: the lines cross near 4 neighbors at any size above.  Quantized, whose decoding a path
+        //! repeats at every node: 330,000 299/148, 326/154, 337/163, 423/165; 990,000 617/373, 675/387,
+        //! 726/397, 998/409.
         static constexpr unsigned int kRopeFronts = 1u << 18;
         //! Queries up to which four waves serve 64, 32, 16 or 4 queries together: one wave's chain of
         //! steps takes longer than the chip needs for all of them.  Exact count and fill of 10,000
