@@ -478,7 +478,7 @@ class LBVHTraverser : public Tunable<unsigned int>
                 }
             }
 
-        //! Wave walk: defined for ExactSphereQueryOp only.
+        //! Bucket records: both sphere queries (exact boxes, the Wave variant: ExactSphereQueryOp only).
         template<class QueryOpT, class OutputOpT, class TranslateOpT, class TransformOpT>
         void traverse_wave(const LaunchParameters& params, const LBVH& lbvh, const QueryOpT& query, const OutputOpT& out,
                            const TranslateOpT& images, const TransformOpT& transform, const unsigned int* order)
@@ -542,18 +542,21 @@ class LBVHTraverser : public Tunable<unsigned int>
         static constexpr unsigned int kTeamQueries = 1u << 16;
         static constexpr unsigned int kFrontsOnly = 1u << 18;
         //! Tail split (wave::tail_block): per XCD, the last groups of 256 queries run as m_tail_split
-        //! blocks each, so that the waves that start last are shorter.  Up to kAllSplit queries, which
-        //! leave wave slots free, all groups do (64 per XCD), up to kHalfSplit 32 of each XCD, above it
-        //! 16.  Exact count and fill in us with 0, 16, 32 and 64 groups (27 images): 100,000 points
-        //! 89/136, 76/116, 72/113 and 73/116; 131,071 92/140, 87/138, 82/131 and 81/125; 200,000
-        //! 148/214, 119/180, 145/225 and 143/232; 300,007 212/322, 206/287, 206/293 and 207/304; 500,000
-        //! 257/374, 236/359, 247/377 and 253/385; 10^6 with 0, 16 and 32 356/594, 348/581 and 358/597.
-        //! Without images: 70,000 points 70/94, 62/84, 59/83 and 54/76; 131,071 76/104, 74/106, 69/100
-        //! and 72/100.  16 groups in four blocks: 300,007 197/293, 500,000 233/355, 200,000 135/206.
+        //! blocks each, so that the waves that start last are shorter.  An XCD holds 128 of the front
+        //! walk's blocks at once: all groups are split while that leaves slots free (up to kAllSplit
+        //! queries), 32 of each XCD as long as the launch is one round then, too (96 + 32 blocks:
+        //! kHalfSplit), above it 16.  Sums of five kinds of count, fill and float count (two radii, with
+        //! and without images, 16 to 48 leaves) in us with 16, 32 and 64 groups: 85,000 points 1365, 1335 and
+        //! 1196; 110,000 1560, 1469, 1442; 120,000 1555, 1471, 1513; 131,072 1645, 1521, 1584; 140,000 1709,
+        //! 1705, 1976; 165,000 1876, 1811, 2211; 180,000 1997, 1890, 2310; 200,000 2032, 2306, 2477; 230,000
+        //! 2386, 2608, 2742; 262,144 2792, 2900, 2964.  Exact count and fill, 500,000 points, with 0, 16 and
+        //! 32: 257/374, 236/359, 247/377; 10^6 356/594, 348/581, 358/597.
+        //! The walk by one rope path per wave (256 blocks per XCD) takes 32 for any number: 10^6 points
+        //! 452 us without, 438 with them.
         unsigned int m_tail_groups = 32;
         unsigned int m_tail_split = 2;
         bool m_tail_set = false;        //!< by setTailSplit: kept for any number of queries
-        static constexpr unsigned int kAllSplit = 3u << 15, kAllSplitGroups = 64, kHalfSplit = 1u << 17, kTailGroups = 16;
+        static constexpr unsigned int kAllSplit = 7u << 14, kAllSplitGroups = 64, kHalfSplit = 3u << 16, kTailGroups = 16;
 
     public:
         //! Leaves per bucket of the wave variant (1..64); takes effect at the next compression.
@@ -565,9 +568,10 @@ class LBVHTraverser : public Tunable<unsigned int>
             }
         unsigned int getBucketSize() const { return m_bucket; }
 
-        //! Tail split of the front walk: per XCD, the last
-        //! `groups` groups of 256 queries run as `split` blocks of 256/split queries each, so the
-        //! waves that start last are shorter (groups = 0: one block per group).
+        //! Tail split of launches of more than kTeamQueries queries: per XCD, the last `groups` groups of
+        //! 256 queries run as `split` blocks of 256/split queries each, so the waves that start last are
+        //! shorter (groups = 0: one block per group).  Kept for any number of queries from then on; before,
+        //! the front walk splits by the number of queries and getTailGroups() is what the other walk takes.
         void setTailSplit(unsigned int groups, unsigned int split)
             {
             if (split != 1 && split != 2 && split != 4) throw std::invalid_argument("the tail split must be 1, 2 or 4");
