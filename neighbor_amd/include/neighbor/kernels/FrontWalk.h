@@ -37,8 +37,9 @@ constexpr unsigned int kStack = 192;        //!< entries of the wave's front
 //! 31 position bits at most) each add one entry there.
 constexpr unsigned int kReserve = 64;
 constexpr unsigned int kList = 128;         //!< buckets found and not yet tested
-//! Hits written at once: the most that leaves four workgroups of 256 threads their LDS (exact fill of
-//! 10^6 points, 78 neighbors each, 595 us against 610 with 512; of clustered rows 2895 against 2952).
+//! Hits written at once: the most that leaves four workgroups of lbvh_traverse_front their LDS (exact
+//! fill of 10^6 points, 78 neighbors each, 595 us against 610 with 512; of clustered rows 2895 against
+//! 2952).  Of lbvh_traverse_team, whose blocks hold the team's words, too, three fit (42 KB each).
 constexpr unsigned int kHits = 1024;
 constexpr unsigned int kLeafStride = 68;    //!< floats between a batch's component rows (bank spread)
 constexpr unsigned int kRun = 32;           //!< leaves from which a node is walked into (sources with kFirst)
@@ -1461,7 +1462,7 @@ lbvh_traverse_wave(const OutputOpT out,
 //! lbvh_traverse_front with the four waves of a block for the same `per` (4, 16, 32 or 64) queries:
 //! launches of few queries, whose time is that of one wave's own chain of steps.
 template<class SrcT, class OutputOpT, class QueryOpT, class TranslateOpT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(std::is_same<OutputOpT, CountNeighborsOp>::value ? 4 : 3, 8)))
 lbvh_traverse_team(const OutputOpT out,
                    SrcT src,
                    const float3* __restrict__ root_lo,
