@@ -122,8 +122,8 @@ int nb_traverser_set_variant(nb_traverser* trav, int variant);
  * setup.  (No reference counterpart.) */
 int nb_traverser_set_bucket_size(nb_traverser* trav, uint32_t bucket);
 
-/* Launch shape of traversals of more than 65,536 queries (nb_traverse_*; not _rows_placed, whose
- * blocks serve whole groups): per XCD, the last `groups` groups of 256 queries run as `split`
+/* Launch shape of traversals of more than 65,536 queries (lists, pairs and rows: 49,152;
+ * nb_traverse_*; not _rows_placed, whose blocks serve whole groups): per XCD, the last `groups` groups of 256 queries run as `split`
  * blocks (1, 2 or 4) of 256/split queries each, so the waves that start last in the launch are
  * shorter.  Default 64 groups up to 114,688 queries, 32 up to 196,608, 16 above (32 for
  * walks by one rope path per wave), split 2; groups = 0: one block per group.

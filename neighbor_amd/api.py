@@ -223,7 +223,7 @@ class LBVHTraverser:
         call("nb_traverser_set_bucket_size", self._h, int(bucket))
 
     def set_tail_split(self, groups: int, split: int = 2) -> None:
-        """Launch shape of traversals of more than 65,536 queries: per XCD, the last `groups` groups
+        """Launch shape of traversals of more than 65,536 queries (lists and rows: 49,152): per XCD, the last `groups` groups
         of 256 queries run as `split` (1, 2 or 4) smaller blocks (default 64 up to 114,688
         queries, 32 up to 196,608, 16 above, and 2; 32 for walks by one rope path per wave); groups 0 =
         one block per group.  Results do not depend on it."""

@@ -351,9 +351,8 @@ class LBVHTraverser : public Tunable<unsigned int>
             constexpr bool teams = !placed && (gpu::kernel::front::Rows<OutputOpT>::kOn || std::is_same<OutputOpT, CountNeighborsOp>::value);
             const unsigned int n = query.size();
             if constexpr (teams)
-                if (n <= kTeamQueries)
+                if (const unsigned int per = teamSize(std::is_same<OutputOpT, CountNeighborsOp>::value, n))
                     {
-                    const unsigned int per = n <= kTeamQueries / 16u ? 4u : n <= kTeamQueries / 4u ? 16u : n <= kTeamQueries / 2u ? 32u : 64u;
                     hipLaunchKernelGGL((gpu::kernel::lbvh_traverse_team<SourceT, OutputOpT, QueryOpT, TranslateOpT>),
                                        dim3(div_up(n, per)), dim3(256), 0, params.stream, out, src, m_lbvh_lo.get(), m_lbvh_hi.get(),
                                        m_bins.get(), m_root, query, images, order, n_nodes, per);
@@ -533,13 +532,28 @@ class LBVHTraverser : public Tunable<unsigned int>
         //! repeats at every node: 330,000 299/148, 326/154, 337/163, 423/165; 990,000 617/373, 675/387,
         //! 726/397, 998/409.
         static constexpr unsigned int kRopeFronts = 1u << 18;
-        //! Queries up to which four waves serve 64, 32, 16 or 4 queries together: one wave's chain of
-        //! steps takes longer than the chip needs for all of them.  Exact count and fill of 10,000
-        //! points (27 images): 82 and 115 us with a wave per 64 queries, 48 and 61 with teams for
-        //! 16; of 131,071 points (no images) 90 and 125 us with waves, 201 and 229 with teams.  Teams
-        //! for 16 and for 4: 1000 points 35 and 47 us, 29 and 38; 4000 points 56 and 72, 45 and 56;
-        //! 8000 points 48 and 65, 62 and 77.
-        static constexpr unsigned int kTeamQueries = 1u << 16;
+        //! Queries that a team of four waves serves together (0: one wave per 64).
+        /*!
+         * One wave's chain of steps takes longer than the chip needs for few queries.  Exact count and fill
+         * of 10,000 points (27 images): 82 and 115 us with a wave per 64 queries, 48 and 61 with teams for
+         * 16; of 131,071 points (no images) 90 and 125 us with waves, 201 and 229 with teams.  Teams for 16
+         * and for 4: 1000 points 35 and 47 us, 29 and 38; 4000 points 56 and 72, 45 and 56; 8000 points 48
+         * and 65, 62 and 77.
+         * The lines lie where a launch fills the chip's round: 1024 blocks that count, 768 of 42 KB of LDS
+         * that write rows; a second round that is nearly empty takes as long as the first.  Fills (27 images,
+         * 79 neighbors, 48 leaves per bucket) by the smaller team and by the next: 12,288 at most in one
+         * round: 13,000 63/53 us, 16,384 76/55; 24,576: 25,000 117/133 (16 leaves; 87/82), 28,000 136/142
+         * (102/88), 32,768 169/155 (115/94): up to 28,672; 49,152: 50,000 145/128, 56,000 151/121, 65,536
+         * 148/108 (no images 125/93; a rope path per wave took 105).  For 4 and 16: 4096 points 60/62, with
+         * 16 leaves 74/108.
+         */
+        static unsigned int teamSize(const bool count, const unsigned int n)
+            {
+            if (n <= (1u << 12)) return 4u;
+            if (n <= (count ? 4u << 12 : 3u << 12)) return 16u;
+            if (n <= (count ? 8u << 12 : 7u << 12)) return 32u;
+            return n <= (count ? 16u << 12 : 12u << 12) ? 64u : 0u;
+            }
         static constexpr unsigned int kFrontsOnly = 1u << 18;
         //! Tail split (wave::tail_block): per XCD, the last groups of 256 queries run as m_tail_split
         //! blocks each, so that the waves that start last are shorter.  An XCD holds 128 of the front
@@ -568,7 +582,7 @@ class LBVHTraverser : public Tunable<unsigned int>
             }
         unsigned int getBucketSize() const { return m_bucket; }
 
-        //! Tail split of launches of more than kTeamQueries queries: per XCD, the last `groups` groups of
+        //! Tail split of launches without teams (teamSize: more than 65,536 counts, 49,152 rows): per XCD, the last `groups` groups of
         //! 256 queries run as `split` blocks of 256/split queries each, so the waves that start last are
         //! shorter (groups = 0: one block per group).  Kept for any number of queries from then on; before,
         //! the front walk splits by the number of queries and getTailGroups() is what the other walk takes.

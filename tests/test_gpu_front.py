@@ -492,3 +492,36 @@ def test_scattered_teams(nb, orc, nq, images):
     assert np.array_equal(rows[0][0], rows[1][0]) and np.array_equal(rows[0][1], rows[1][1])
     ref = orc.exact_bruteforce(pts, sph[:2000], imgs.astype(np.float64) if images else np.zeros((1, 3)), pairs=False)
     assert np.array_equal(rows[0][0][:2000].view(np.uint32), ref["counts"])
+
+
+@pytest.mark.parametrize("n", [4096, 4097, 12288, 12289, 28672, 28673, 49152, 49153])
+def test_rows_by_team_size(nb, n):
+    """Rows and lists on both sides of the lines between teams, and between teams and waves, equal the
+    one-by-one emission of a path per query."""
+    import torch
+    from neighbor_amd.api import exact_rows, exclusive_scan
+    from neighbor_amd.workloads import images27
+    rng = np.random.default_rng(n + 9)
+    nt = 300000     # exact queries over float rope records take a path each above 2^18
+    pts, L = points_of(nt, rng, "uniform")
+    d_pts = torch.from_numpy(pts).cuda()
+    lb = nb.LBVH()
+    lb.build(d_pts, [0, 0, 0], [L] * 3)
+    sph = torch.cat([d_pts, torch.full((nt, 1), 1.2, device="cuda")], 1).contiguous()
+    img = torch.from_numpy(images27(L, dtype=np.float64)).cuda()
+    paths = nb.LBVHTraverser(variant=nb.NB_VARIANT_FLOAT_ROPE_EXACT)
+    every = paths.exact_count(lb, sph, d_pts, images=img)
+    all_start = exclusive_scan(every)
+    all_neigh = torch.empty(int(all_start[-1]), dtype=torch.int32, device="cuda")
+    exact_rows(paths, lb, sph, d_pts, all_start, every, all_neigh, images=img)
+    few = sph[:n].contiguous()
+    total = int(all_start[n])
+    for variant in (nb.NB_VARIANT_WAVE, nb.NB_VARIANT_FLOAT_ROPE_EXACT):
+        tr = nb.LBVHTraverser(variant=variant)
+        neigh = torch.full((total,), -1, dtype=torch.int32, device="cuda")
+        got = exact_rows(tr, lb, few, d_pts, all_start[:n].contiguous(), every[:n].contiguous(), neigh, images=img)
+        assert torch.equal(got, every[:n]) and torch.equal(neigh, all_neigh[:total])
+    counts = nb.LBVHTraverser().count(lb, sph, images=img.float())
+    lst, nn = nb.LBVHTraverser().neighbor_list(lb, few, 24, images=img.float())
+    want, _ = nb.LBVHTraverser(variant=nb.NB_VARIANT_FLOAT_ROPE).neighbor_list(lb, sph, 24, images=img.float())
+    assert torch.equal(nn, counts[:n]) and torch.equal(lst, want[:n])
