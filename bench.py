@@ -55,8 +55,8 @@ def parse():
     ap.add_argument("--bucket", type=int, default=48, help="leaves per bucket (wave variants)")
     ap.add_argument("--block", type=int, default=256)
     ap.add_argument("--tail-groups", type=int, default=None,
-                    help="exact wave walks: last groups of 256 queries per XCD run as split blocks "
-                         "(default: the library's, 32)")
+                    help="traversals: last groups of 256 queries per XCD run as split blocks "
+                         "(default: the library's, by the number of queries)")
     ap.add_argument("--tail-split", type=int, default=2, help="blocks per split group (1, 2 or 4)")
     ap.add_argument("--pad", type=int, default=8, help="capacity rows: predicted count + pad")
     ap.add_argument("--quantile", type=float, default=0.999,

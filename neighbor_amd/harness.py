@@ -11,7 +11,8 @@ For each frame, starting from 0, as the reference harness does:
 - one sphere of radius rcut per particle, listed in the tree's primitive (Morton) order, and
   the 27 periodic images listed center first (lbvh_benchmark.cc:183-207);
 - the count traversal of the reference's structure (quantized per-thread ropes, SphereQueryOp),
-  its block size tuned the same way, then the median of 5 x K calls.
+  its block size tuned the same way, then the median of 5 x K calls (the walk by node fronts
+  takes blocks of 256 threads whatever is asked for, so here the tuning is the protocol's alone).
 
 The output table keeps the reference's columns (frame, build (ms), traverse (ms)) and adds this
 library's exact wave walk (FP64 pair test) as a fourth column.

@@ -12,8 +12,9 @@
 // ExactSphereQueryOp (with the float SphereQueryOp it reports fewer, tighter hits than the
 // reference); Wave (ExactSphereQueryOp only) exact-box records with bucket leaves; WaveQuantized
 // the same over decoded quantized boxes, for SphereQueryOp (results identical to Quantized) and
-// ExactSphereQueryOp.  Both queries walk by node fronts (kernels/FrontWalk.h); other query ops, and
-// many exact queries over rope records (kRopeFronts), take one rope path per query.
+// ExactSphereQueryOp.  Both queries walk by node fronts (kernels/FrontWalk.h), many exact queries over
+// bucket records by one rope path per wave (kernels/WaveWalk.h, sparseLimit); other query ops, and
+// many exact queries over float rope records (kRopeFronts), take one rope path per query.
 #ifndef NEIGHBOR_LBVH_TRAVERSER_H_
 #define NEIGHBOR_LBVH_TRAVERSER_H_
 
@@ -416,8 +417,8 @@ class LBVHTraverser : public Tunable<unsigned int>
          *    164/164, 237/259, 10^6 306/384, 370/442, 531/550; 16 leaves: 10^6 366/386, 452/484, 666/634.
          *    27 images, 64 leaves: 700,000 295/311, 343/349, 442/418, 10^6 374/433, 453/487, 611/601; 32
          *    leaves: 10^6 398/403, 469/472, 641/586, 2 10^6 683/773, 842/849, 1268/1380.
-         * Left: rows with images of sparse queries (5 neighbors, 10^6, 64 leaves: 314/403), and rows of
-         * 300,000 dense ones with images (64 leaves 254/278).
+         * Left, with images: sparse queries (5 neighbors, 10^6: rows with 48 leaves 326/380, counts with
+         * 64 leaves 263/317), and rows of 300,000 dense ones (64 leaves 254/278).
          */
         static float sparseLimit(const bool rows, const unsigned int n, const unsigned int bucket, const unsigned int images)
             {
